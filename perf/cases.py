@@ -103,8 +103,8 @@ def draw(rng):
                 batch, m, n, k = 1, _size(rng, 16, 256), _size(rng, 64, 512), _size(rng, 8192, 131072)
             else:
                 m, n, k = _size(rng, 1, 4096), _size(rng, 64, 6144), _size(rng, 64, 6144)
-            if kind == "a16":
-                m = max(m, 9)
+            if kind == "a16":  # its kernels take whole multiples of these only
+                m, n, k = max(1, round(m / 64)) * 64, max(1, round(n / 64)) * 64, max(1, round(k / 32)) * 32
             if batch * m * n * k <= 4096 ** 3:
                 break
         plain = kind == "a16"  # f16 activations take no epilogue
