@@ -40,31 +40,11 @@ namespace {
 template <int DH> constexpr int flash_parts() { return ta_flash_parts(DH); }     // KP
 template <int DH> constexpr int flash_qblocks() { return ta_flash_qblocks(DH); } // QB
 constexpr float kNegMax = -3.402823466e38f;
-
-template <bool F16> TA_DEVICE f32x4 load4(const void *base, uint64_t i) {
-  if constexpr (F16) {
-    const f16x4 h = *reinterpret_cast<const f16x4 *>(static_cast<const _Float16 *>(base) + i);
-    return f32x4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
-  } else {
-    return *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + i);
-  }
-}
-// Cache loads in storage type; widened to f32 only when written to LDS,
-// so a prefetch does not wait for its data at the load.
-template <bool F16> TA_DEVICE auto load_raw(const void *base, uint64_t i) {
-  if constexpr (F16)
-    return *reinterpret_cast<const f16x4 *>(static_cast<const _Float16 *>(base) + i);
-  else
-    return *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + i);
-}
-template <bool F16> TA_DEVICE auto load_raw1(const void *base, uint64_t i) {
-  if constexpr (F16)
-    return static_cast<const _Float16 *>(base)[i];
-  else
-    return static_cast<const float *>(base)[i];
-}
-TA_DEVICE f32x4 widen(f32x4 v) { return v; }
-TA_DEVICE f32x4 widen(f16x4 h) { return f32x4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]}; }
+constexpr float kMasked = -__builtin_inff();
+constexpr float kMinScale = 1.17549435e-38f; // 2^-126
+// f16-cache kernels: a row's probabilities stay below 2^kSlack, and are
+// scaled by kProbScale so that their f16 pieces reach down to 2^-35 of it.
+constexpr float kSlack = 4.0f, kProbScale = 2048.0f;
 
 template <bool F16> TA_DEVICE void store4(void *base, uint64_t i, f32x4 v) {
   if constexpr (F16) {
@@ -75,7 +55,82 @@ template <bool F16> TA_DEVICE void store4(void *base, uint64_t i, f32x4 v) {
   }
 }
 
-template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArgs &p) {
+// (head, query tile) of this workgroup.  Consecutive workgroups go to the 8
+// XCDs in turn; with a multiple of 8 heads, all tiles of a head run on one
+// XCD (its L2 keeps that head's K/V).  Tiles start longest first over all
+// heads of an XCD: the last tile of a causal prompt has q_tiles times the
+// first one's keys, and head by head the second half of the heads started
+// its longest tiles when the first had drained (2048 tokens, 32 heads, dh
+// 128: SQ_BUSY_CU_CYCLES two thirds of the launch).
+TA_DEVICE void flash_work(const FlashArgs &p, uint32_t &head, uint32_t &tile) {
+  uint32_t i = blockIdx.x, first = 0, count = p.heads;
+  if (p.heads % 8u == 0u) {
+    count = p.heads >> 3;
+    first = (i & 7u) * count;
+    i >>= 3;
+  }
+  head = first + i % count;
+  tile = p.q_tiles - 1u - i / count;
+}
+
+// Maximum over the two lanes (halves of the wave) that share a query row.
+TA_DEVICE float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// One wave's 32 query rows in plain f32 arithmetic, for rows whose result
+// is not finite: an infinite operand must not meet the zero pieces of a
+// split one (inf * 0), so these rows are computed again with whole values.
+template <int DH, bool IO16>
+TA_DEVICE void flash_rows_plain(const FlashArgs &p, uint32_t head, uint32_t kv_head, uint32_t row0,
+                                uint32_t lane) {
+  const _Float16 *kt = static_cast<const _Float16 *>(p.kt) + (uint64_t)kv_head * DH * p.t_max;
+  const _Float16 *vv = static_cast<const _Float16 *>(p.v) + (uint64_t)kv_head * p.t_max * DH;
+  const float scale2 = p.scale * 1.44269504088896340736f;
+  for (uint32_t row = row0; row < min(row0 + 32u, p.t_q); ++row) {
+    const uint32_t valid = min(min(p.kv_len, p.pos_base + row + 1u), p.t_max);
+    const uint64_t qbase = (uint64_t)head * p.q_head_stride + (uint64_t)row * p.q_row_stride;
+    auto score = [&](uint32_t key) {
+      float acc = 0.0f;
+      for (uint32_t d = 0; d < (uint32_t)DH; ++d)
+        acc = fmaf(IO16 ? (float)static_cast<const _Float16 *>(p.q)[qbase + d]
+                        : static_cast<const float *>(p.q)[qbase + d],
+                   (float)kt[(uint64_t)d * p.t_max + key], acc);
+      return acc * scale2;
+    };
+    float m = kNegMax;
+    for (uint32_t key = lane; key < valid; key += 64u)
+      m = fmaxf(m, score(key));
+    for (int x = 32; x > 0; x >>= 1)
+      m = fmaxf(m, __shfl_xor(m, x));
+    float l = 0.0f, acc[DH / 64];
+    for (int i = 0; i < DH / 64; ++i)
+      acc[i] = 0.0f;
+    for (uint32_t k0 = 0; k0 < valid; k0 += 64u) {
+      const float pk = k0 + lane < valid ? exp2f(score(k0 + lane) - m) : 0.0f;
+      l += pk;
+      for (uint32_t k = 0; k < min(64u, valid - k0); ++k) {
+        const float w = __shfl(pk, (int)k);
+        for (int i = 0; i < DH / 64; ++i)
+          acc[i] = fmaf(w, (float)vv[(uint64_t)(k0 + k) * DH + i * 64 + lane], acc[i]);
+      }
+    }
+    for (int x = 32; x > 0; x >>= 1)
+      l += __shfl_xor(l, x);
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const uint64_t obase = (uint64_t)head * p.o_head_stride + (uint64_t)row * p.o_row_stride;
+    for (int i = 0; i < DH / 64; ++i) {
+      const uint64_t at = obase + i * 64 + lane;
+      if constexpr (IO16)
+        static_cast<_Float16 *>(p.out)[at] = (_Float16)(acc[i] * inv);
+      else
+        static_cast<float *>(p.out)[at] = acc[i] * inv;
+    }
+  }
+}
+
+template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
   constexpr int KP = flash_parts<DH>();  // key parts
   constexpr int QB = flash_qblocks<DH>(); // 32-row query blocks
   constexpr int kBQ = 32 * QB;           // query rows per workgroup
@@ -94,14 +149,8 @@ template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArg
   const uint32_t qb = wave % QB, kh = wave / QB;
   const uint32_t j = lane & 31u, h = lane >> 5;
 
-  // Workgroups of one head run on one XCD (its L2 keeps that head's K/V);
-  // within a head the longest (latest) query tiles start first.
-  const uint32_t total = p.q_tiles * p.heads;
-  uint32_t pidx = blockIdx.x;
-  if (total % 8u == 0u)
-    pidx = (blockIdx.x & 7u) * (total >> 3) + (blockIdx.x >> 3);
-  const uint32_t head = pidx / p.q_tiles;
-  const uint32_t tile = p.q_tiles - 1u - pidx % p.q_tiles;
+  uint32_t head, tile;
+  flash_work(p, head, tile);
 
   const uint32_t q0 = tile * kBQ;
   const uint32_t qrow = q0 + qb * 32u + j;
@@ -120,7 +169,7 @@ template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArg
                            (uint64_t)min(qrow, p.t_q - 1u) * p.q_row_stride + h * HALF;
 #pragma unroll
     for (int s = 0; s < HALF; s += 4) {
-      const f32x4 v = load4<IO16>(p.q, qbase + s);
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(p.q) + qbase + s);
       qreg[s] = v[0];
       qreg[s + 1] = v[1];
       qreg[s + 2] = v[2];
@@ -142,8 +191,8 @@ template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArg
   // is computed: ksh[d][c] = Kt[d][k0 + c] in KC four-key chunks per row,
   // vsh[r][d] = V[k0 + r][d].
   constexpr int NCH = DH * kBK / 4 / kFlashThreads;
-  using Raw = typename std::conditional<KV16, f16x4, f32x4>::type; // widened at the LDS store
-  Raw kreg[NCH], vreg[NCH];
+  const float *kt = static_cast<const float *>(p.kt), *vv = static_cast<const float *>(p.v);
+  f32x4 kreg[NCH], vreg[NCH];
   auto load_tile = [&](uint32_t k0) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
@@ -151,18 +200,18 @@ template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArg
       const uint32_t d = c / KC, key = k0 + (c % KC) * 4u;
       const uint64_t src = kt_base + (uint64_t)d * p.t_max + key;
       if (kt_vec && key + 3u < stage_end) {
-        kreg[i] = load_raw<KV16>(p.kt, src);
+        kreg[i] = *reinterpret_cast<const f32x4 *>(kt + src);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          kreg[i][e] = key + e < stage_end ? load_raw1<KV16>(p.kt, src + e) : 0;
+          kreg[i][e] = key + e < stage_end ? kt[src + e] : 0.0f;
       }
     }
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const uint32_t c = tid + i * kFlashThreads;
       const uint32_t key = k0 + c / (DH / 4), dc = (c % (DH / 4)) * 4u;
-      vreg[i] = key < stage_end ? load_raw<KV16>(p.v, v_base + (uint64_t)key * DH + dc) : Raw{};
+      vreg[i] = key < stage_end ? *reinterpret_cast<const f32x4 *>(vv + v_base + (uint64_t)key * DH + dc) : f32x4{};
     }
   };
   if (n_tiles > 0)
@@ -178,8 +227,8 @@ template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArg
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const uint32_t c = tid + i * kFlashThreads;
-      *reinterpret_cast<f32x4 *>(ksh + (c / KC) * kBK + (c % KC) * 4u) = widen(kreg[i]);
-      *reinterpret_cast<f32x4 *>(vsh + (c / (DH / 4)) * DH + (c % (DH / 4)) * 4u) = widen(vreg[i]);
+      *reinterpret_cast<f32x4 *>(ksh + (c / KC) * kBK + (c % KC) * 4u) = kreg[i];
+      *reinterpret_cast<f32x4 *>(vsh + (c / (DH / 4)) * DH + (c % (DH / 4)) * 4u) = vreg[i];
     }
     __syncthreads();
     if (t + 1 < n_tiles)
@@ -292,22 +341,465 @@ template <int DH, bool KV16, bool IO16> TA_DEVICE void flash_body(const FlashArg
               acc += mb[((k - 1) * REGS + e) * 64 + lane] * a[k];
             v[r] = acc * inv;
           }
-          store4<IO16>(p.out, obase + b * 32 + 8 * q, v);
+          store4<false>(p.out, obase + b * 32 + 8 * q, v);
         }
     }
   }
 }
 
-} // namespace
+// ---------------------------------------------------------------------
+// f16 caches: both products on v_mfma_f32_32x32x16_f16 (16 times the f32
+// rate), with f32 accuracy kept by splitting the f32 operands into f16
+// pieces whose products with the f16 cache values are exact in the f32
+// accumulator:
+//  * q: as it is when f16; f32 rows are scaled by a power of two (largest
+//    value into [2^14, 2^15)) and split exactly into three pieces;
+//  * probabilities p: two pieces of p * kProbScale (22 bits of every p down
+//    to 2^-18, and 2^-36 absolute below that); the row sum takes the f32 p.
+// Measured against f64 (normal inputs): 1.7e-7 .. 3.5e-7, as the f32 MFMA
+// kernel had.  An infinite operand would meet zero pieces (inf * 0); rows
+// that come out non-finite are computed again by flash_rows_plain.
+//
+// Layout.  K and V tiles stay in LDS as they lie in the caches ([d][key],
+// [key][d]), and both reach the matrix cores through ds_read_b64_tr_b16.
+// Scores are computed transposed (m = key, n = query), so a lane owns one
+// query row and the PV product takes P straight from the score registers:
+// step u pairs registers 8u .. 8u+7 with V rows 16u + 4h + {0..3, 8..11}.
+// Tiles arrive by direct global -> LDS loads into two buffers with one
+// barrier per tile.  The q registers are pinned before the loop: the
+// compiler's own wait for q's loads inside it also waited for the tile in
+// flight (112 -> 94 us at the size below).
+//
+// Split.  Four waves: 2 query blocks x 2 key parts of 32 keys, or 1 x 4
+// for short prompts (twice the workgroups, a quarter of the keys per
+// wave; ta_flash16_rows).  Tiles of 128 rows x 64 keys were slower (102
+// against 94 us): fewer, longer workgroups leave CUs idle at the end.
+//
+// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 73 us
+// here (470 TFLOP/s), kv16 434 -> 98 us; 512 tokens, 4 KV heads, dh 64, f16:
+// 28 -> 10.8 us.  MFMAs are busy 33% and the VALU (exp2, splits) about as
+// long; a wave's two phases overlap only with its SIMD's other wave.
+template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH16 {
+  static constexpr int T = 64 * QB * KP;
+  static constexpr int BQ = 32 * QB;         // query rows per workgroup
+  static constexpr int BK = KP * BKW;        // keys per tile
+  static constexpr int KB = BKW / 32;        // 32-key score blocks per wave
+  static constexpr int KS = DH / 16;         // MFMA k-steps of the score product
+  static constexpr int DB = DH / 32;         // 32-row head-dim blocks of the output
+  static constexpr int QP = IO16 ? 1 : 3;    // f16 pieces of q
+  static constexpr int K_BYTES = DH * BK * 2, STAGE = 2 * K_BYTES;
+  static constexpr int CK = BK / 8, CV = DH / 8; // 16-byte chunks per K / V row
+  static constexpr int LD = K_BYTES / 16 / T;    // direct loads per thread, per operand
+  static constexpr int REGS = DB * 16 + 2;       // merge record per lane: o, m, l
+  static constexpr int MERGE = QB * (KP - 1) * REGS * 64 * 4;
+  static constexpr int SMEM = 2 * STAGE > MERGE ? 2 * STAGE : MERGE;
+  static_assert(LD * T * 16 == K_BYTES && CK >= 8 && CV >= 8, "stages split evenly");
+  static_assert(SMEM <= 160 * 1024, "LDS");
 
-#define TA_FLASH(NAME, DH, KV16, IO16)                                                     \
-  extern "C" __global__ __launch_bounds__(64 * flash_qblocks<DH>() * flash_parts<DH>()) void NAME(FlashArgs p) { \
-    flash_body<DH, KV16, IO16>(p);                                                         \
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+  static TA_DEVICE uint32_t swz(uint32_t row, int chunks) {
+    return chunks >= 16 ? (0xACA60u >> (4u * (row & 3u))) & 15u : 2u * (row & 3u);
+  }
+  // `base` and `lds` are the same in every lane.
+  static TA_DEVICE void load16s(const void *src, uint32_t off, uint32_t lds) {
+    const uint64_t a = reinterpret_cast<uint64_t>(src);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    const uint64_t base = (uint64_t)lo | (uint64_t)hi << 32;
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory", "m0");
+  }
+  // Two transpose reads: rows r .. r + 3 (`lo`) and r' .. r' + 3 (`hi`) of
+  // this lane's column.
+  static TA_DEVICE f16x8 tr(uint32_t lo, uint32_t hi) {
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(uintptr_t)lo);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(uintptr_t)hi);
+    return __builtin_bit_cast(f16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
   }
 
-TA_FLASH(ta_flash_attention_dh64, 64, false, false)
-TA_FLASH(ta_flash_attention_dh128, 128, false, false)
-TA_FLASH(ta_flash_attention_kv16_dh64, 64, true, false)
-TA_FLASH(ta_flash_attention_kv16_dh128, 128, true, false)
-TA_FLASH(ta_flash_attention_io16_dh64, 64, true, true)
-TA_FLASH(ta_flash_attention_io16_dh128, 128, true, true)
+  static TA_DEVICE void run(const FlashArgs &p) {
+    __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t qb = wave % QB, kh = wave / QB;
+    const uint32_t j = lane & 31u, h = lane >> 5;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
+
+    uint32_t head, tile;
+    flash_work(p, head, tile);
+    const uint32_t q0 = tile * BQ, qw0 = q0 + qb * 32u, qrow = qw0 + j;
+    const bool live = qrow < p.t_q;
+    const uint32_t kv_head = head / p.group_size;
+    const uint32_t valid_row = live ? min(p.kv_len, p.pos_base + qrow + 1u) : 0u;
+    const uint32_t last_row = min(q0 + (uint32_t)BQ, p.t_q) - 1u;
+    const uint32_t valid_max = min(p.kv_len, p.pos_base + last_row + 1u);
+    const uint32_t stage_end = min(valid_max, p.t_max);
+    const uint32_t n_tiles = (valid_max + BK - 1u) / BK;
+    // keys every row of this wave attends to / any row of it does
+    const uint32_t wave_all = min(p.kv_len, p.pos_base + qw0 + 1u);
+    const uint32_t wave_any = qw0 < p.t_q ? min(p.kv_len, p.pos_base + min(qw0 + 32u, p.t_q)) : 0u;
+
+    // This lane's q operand: Q[qrow][16 s + 8 h .. + 7] of every step s.
+    f16x8 qf[QP][KS];
+    const float s2 = p.scale * 1.44269504088896340736f, sign = s2 < 0.0f ? -1.0f : 1.0f;
+    float scale2 = s2 * sign; // the sign goes to q
+    {
+      const uint64_t qbase = (uint64_t)head * p.q_head_stride +
+                             (uint64_t)min(qrow, p.t_q - 1u) * p.q_row_stride + h * 8u;
+      if constexpr (IO16) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          qf[0][s] = *reinterpret_cast<const f16x8 *>(static_cast<const _Float16 *>(p.q) + qbase + 16 * s) *
+                     (_Float16)sign;
+      } else {
+        const float *src = static_cast<const float *>(p.q) + qbase;
+        float qmax = 0.0f;
+        f32x4 raw[KS][2];
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            raw[s][i] = *reinterpret_cast<const f32x4 *>(src + 16 * s + 4 * i);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              qmax = fmaxf(qmax, fabsf(raw[s][i][c]));
+          }
+        qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+        // largest |q| of the row into [2^14, 2^15)
+        int e = 15 - __builtin_amdgcn_frexp_expf(qmax);
+        e = qmax > 0.0f ? min(max(e, -100), 100) : 0;
+        const float up = ldexpf(sign, e);
+        scale2 = scale2 * ldexpf(1.0f, -e);
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            float x = raw[s][i / 4][i % 4] * up;
+#pragma unroll
+            for (int q = 0; q < QP; ++q) {
+              qf[q][s][i] = (_Float16)x;
+              x -= (float)qf[q][s][i];
+            }
+          }
+      }
+    }
+
+    // A scale that underflows (or 0) keeps every finite score at 0 and a
+    // masked one (-inf) at -inf.
+    scale2 = scale2 < kMinScale ? kMinScale : scale2;
+    // The loads of q end here: the compiler places its waits before the
+    // first use, and one inside the loop would also wait for the tile in
+    // flight.
+#pragma unroll
+    for (int q = 0; q < QP; ++q)
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        asm volatile("" : "+v"(qf[q][s]));
+
+    f32x16 o[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+      o[b] = f32x16{};
+    float m_run = kNegMax, l_run = 0.0f;
+
+    const _Float16 *kt = static_cast<const _Float16 *>(p.kt) + (uint64_t)kv_head * DH * p.t_max;
+    const _Float16 *vv = static_cast<const _Float16 *>(p.v) + (uint64_t)kv_head * p.t_max * DH;
+    // Stage tile t: K as [d][key], V as [key][d], 16-byte chunks swizzled
+    // within a row.  Whole tiles go through a uniform base and fixed lane
+    // offsets; a tile that runs past the cache clamps every address (its
+    // keys past t_max are masked, its V rows zeroed below).
+    uint32_t koff[LD], voff[LD];
+#pragma unroll
+    for (int i = 0; i < LD; ++i) {
+      const uint32_t q = i * T + tid;
+      uint32_t row = q / CK, c = (q % CK) ^ swz(row, CK);
+      koff[i] = row * p.t_max + 8u * c;
+      row = q / CV, c = (q % CV) ^ swz(row, CV);
+      voff[i] = row * DH + 8u * c;
+    }
+    // K rows that are not whole 16-byte pieces go through registers:
+    // fetched before a tile's compute, written to LDS after it.
+    f16x8 kreg[DIRECT ? 1 : LD];
+    const uint64_t k_left = (uint64_t)(p.heads / p.group_size - kv_head) * DH * p.t_max;
+    auto issue = [&](uint32_t t) __attribute__((always_inline)) {
+      const uint32_t k0 = t * BK;
+      const uint32_t base = __builtin_amdgcn_readfirstlane(lds0 + (t & 1u) * STAGE + wave * 1024u);
+      const _Float16 *ks = kt + k0, *vs = vv + (uint64_t)k0 * DH;
+      const bool whole = k0 + BK <= p.t_max;
+      if constexpr (DIRECT) {
+        if (whole) {
+#pragma unroll
+          for (int i = 0; i < LD; ++i)
+            load16s(ks, koff[i] * 2u, base + i * T * 16u);
+        } else {
+#pragma unroll
+          for (int i = 0; i < LD; ++i) {
+            const uint32_t row = (i * T + tid) / CK, key = k0 + koff[i] - row * p.t_max;
+            load16s(kt, (row * p.t_max + min(key, p.t_max - 8u)) * 2u, base + i * T * 16u);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+          typedef f16x8 f16x8u __attribute__((aligned(2)));
+          const uint32_t q = i * T + tid, row = q / CK, c = (q % CK) ^ swz(row, CK);
+          const uint64_t at = (uint64_t)row * p.t_max + k0 + 8u * c;
+          if (at + 8u <= k_left) {
+            kreg[i] = *reinterpret_cast<const f16x8u *>(kt + at);
+          } else {
+#pragma unroll
+            for (int x = 0; x < 8; ++x)
+              kreg[i][x] = at + x < k_left ? kt[at + x] : (_Float16)0.0f;
+          }
+        }
+      }
+      if (whole) {
+#pragma unroll
+        for (int i = 0; i < LD; ++i)
+          load16s(vs, voff[i] * 2u, base + K_BYTES + i * T * 16u);
+      } else {
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+          const uint32_t row = (i * T + tid) / CV;
+          load16s(vs, (voff[i] + (min(k0 + row, p.t_max - 1u) - k0 - row) * DH) * 2u,
+                  base + K_BYTES + i * T * 16u);
+        }
+      }
+    };
+    auto commit = [&](uint32_t t) __attribute__((always_inline)) {
+      if constexpr (!DIRECT) {
+#pragma unroll
+        for (int i = 0; i < LD; ++i)
+          *reinterpret_cast<f16x8 *>(smem + (t & 1u) * STAGE + (i * T + tid) * 16u) = kreg[i];
+      }
+    };
+
+    // Per-lane LDS read offsets (transpose reads: group g of 16 lanes, t).
+    const uint32_t g = lane >> 4, t16 = lane & 15u;
+    uint32_t k_off[KB], v_off[DB];
+    {
+      const uint32_t row = 8u * (g >> 1) + (t16 >> 2);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const uint32_t col = kh * BKW + kb * 32u + 16u * (g & 1u) + 4u * (t16 & 3u);
+        k_off[kb] = row * (BK * 2) + 16u * ((col >> 3) ^ swz(row, CK)) + (col & 7u) * 2u;
+      }
+      const uint32_t vrow = kh * BKW + 4u * (g >> 1) + (t16 >> 2);
+#pragma unroll
+      for (int b = 0; b < DB; ++b) {
+        const uint32_t col = b * 32u + 16u * (g & 1u) + 4u * (t16 & 3u);
+        v_off[b] = K_BYTES + vrow * (DH * 2) + 16u * ((col >> 3) ^ swz(vrow, CV)) + (col & 7u) * 2u;
+      }
+    }
+
+    if (n_tiles > 0) {
+      issue(0);
+      commit(0);
+    }
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+      const uint32_t k0 = t * BK;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads(); // tile t landed; every wave is done with tile t - 1
+      if (t + 1 < n_tiles)
+        issue(t + 1);
+      if (k0 + BK > stage_end) {
+        // rows of V at or past the frontier become zeros (unwritten cache
+        // memory may hold anything, and 0 * inf is not 0)
+        const uint32_t first = stage_end - min(stage_end, k0);
+        char *vs = smem + (t & 1u) * STAGE + K_BYTES;
+        for (uint32_t i = first * (DH * 2 / 16) + tid; i < (uint32_t)(BK * DH * 2 / 16); i += T)
+          *reinterpret_cast<f32x4 *>(vs + i * 16u) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        __syncthreads();
+      }
+      const uint32_t kw0 = k0 + kh * BKW;
+      if (kw0 >= wave_any) { // no row of this wave attends to these keys
+        if (t + 1 < n_tiles)
+          commit(t + 1);
+        continue;
+      }
+      const uint32_t st = lds0 + (t & 1u) * STAGE;
+
+      f32x16 s[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        s[kb] = f32x16{};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const uint32_t at = st + k_off[kb] + ks * 16 * (BK * 2);
+          const f16x8 a = tr(at, at + 4 * (BK * 2));
+#pragma unroll
+          for (int q = 0; q < QP; ++q)
+            s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[q][ks], s[kb], 0, 0, 0);
+        }
+
+      float tmax = kNegMax;
+      if (kw0 + BKW > wave_all) {
+        const uint32_t kbase = kw0 + 4u * h;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const uint32_t key = kbase + kb * 32u + 8u * (e / 4) + (e % 4);
+            s[kb][e] = key < valid_row ? s[kb][e] : kMasked;
+          }
+      }
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          tmax = fmaxf(tmax, s[kb][e]);
+      tmax = fmaxf(half_max(tmax) * scale2, kNegMax);
+      // The reference point moves only when a row's maximum has outgrown it
+      // by 2^kSlack (probabilities stay below 2^kSlack): with 32 rows in a
+      // wave some row finds a new maximum in nearly every tile, and scaling
+      // the output for it was a third of the softmax's instructions.
+      if (__any(tmax > m_run + kSlack)) {
+        const float m_new = fmaxf(m_run, tmax);
+        const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= corr;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            o[b][e] *= corr;
+      }
+      float psum = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][e], scale2, -m_run));
+          psum += pv;
+          s[kb][e] = pv * kProbScale;
+        }
+      l_run += psum;
+
+      // O^T += V^T P^T: step u of a 32-key block pairs P registers 8u..8u+7
+      // (keys 16u + 4h + 0..3 and 16u + 8 + 4h + 0..3) with the same V rows.
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f16x8 hi, lo;
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+            const float x = s[kb][8 * u + e], y = s[kb][8 * u + e + 1];
+            f16x2 a = {(_Float16)x, (_Float16)y};
+            asm("" : "+v"(a)); // widen from the packed pair
+            hi[e] = a[0];
+            hi[e + 1] = a[1];
+            lo[e] = (_Float16)(x - (float)a[0]);
+            lo[e + 1] = (_Float16)(y - (float)a[1]);
+          }
+#pragma unroll
+          for (int b = 0; b < DB; ++b) {
+            const uint32_t at = st + v_off[b] + (kb * 32 + u * 16) * (DH * 2);
+            const f16x8 a = tr(at, at + 8 * (DH * 2));
+            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi, o[b], 0, 0, 0);
+            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo, o[b], 0, 0, 0);
+          }
+        }
+      if (t + 1 < n_tiles)
+        commit(t + 1);
+    }
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        o[b][e] *= 1.0f / kProbScale;
+
+    float m = m_run, l = l_run, a0 = 1.0f;
+    float mp[KP], a[KP];
+    float *mb = reinterpret_cast<float *>(smem) + qb * ((KP - 1) * REGS * 64);
+    if constexpr (KP > 1) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (kh != 0u) {
+        float *rec = mb + (kh - 1u) * (REGS * 64);
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            rec[(b * 16 + e) * 64 + lane] = o[b][e];
+        rec[(DB * 16) * 64 + lane] = m_run;
+        rec[(DB * 16 + 1) * 64 + lane] = l_run;
+      }
+      __syncthreads();
+      if (kh != 0u)
+        return;
+#pragma unroll
+      for (int k = 1; k < KP; ++k) {
+        mp[k] = mb[((k - 1) * REGS + DB * 16) * 64 + lane];
+        m = fmaxf(m, mp[k]);
+      }
+      a0 = __builtin_amdgcn_exp2f(m_run - m);
+      l = l_run * a0;
+#pragma unroll
+      for (int k = 1; k < KP; ++k) {
+        a[k] = __builtin_amdgcn_exp2f(mp[k] - m);
+        l += mb[((k - 1) * REGS + DB * 16 + 1) * 64 + lane] * a[k];
+      }
+    }
+    l += __shfl_xor(l, 32);
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    bool finite = true;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        float acc = o[b][e] * a0;
+        if constexpr (KP > 1) {
+#pragma unroll
+          for (int k = 1; k < KP; ++k)
+            acc += mb[((k - 1) * REGS + b * 16 + e) * 64 + lane] * a[k];
+        }
+        o[b][e] = acc * inv;
+        finite = finite && __builtin_isfinite(o[b][e]);
+      }
+    if (live) {
+      const uint64_t obase =
+          (uint64_t)head * p.o_head_stride + (uint64_t)qrow * p.o_row_stride + 4u * h;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          store4<IO16>(p.out, obase + b * 32 + 8 * q,
+                       f32x4{o[b][4 * q], o[b][4 * q + 1], o[b][4 * q + 2], o[b][4 * q + 3]});
+    }
+    if (__any(live && !finite))
+      flash_rows_plain<DH, IO16>(p, head, kv_head, qw0, lane);
+  }
+};
+
+} // namespace
+
+#define TA_FLASH(DH)                                                                        \
+  extern "C" __global__ __launch_bounds__(ta_flash_threads(DH)) void                         \
+  ta_flash_attention_dh##DH(FlashArgs p) {                                                   \
+    flash_body<DH>(p);                                                                       \
+  }
+TA_FLASH(64)
+TA_FLASH(128)
+
+// f16 caches (kv16: f32 q/out, io16: f16 q/out): 64-row and 32-row query
+// tiles, and `_any` forms for caches whose K rows are not whole 16-byte
+// pieces.  At least two waves per SIMD share the registers.
+#define TA_FLASH_H16(SYM, DH, IO16, ROWS, DIRECT)                                            \
+  extern "C" __global__ __launch_bounds__(256, 2) void SYM(FlashArgs p) {                    \
+    FlashH16<DH, IO16, DIRECT, ROWS / 32, 128 / ROWS, 32>::run(p);                           \
+  }
+#define TA_FLASH_H16_FAMILY(DH, ROWS)                                                        \
+  TA_FLASH_H16(ta_flash_attention_kv16_dh##DH##_r##ROWS, DH, false, ROWS, true)              \
+  TA_FLASH_H16(ta_flash_attention_kv16_dh##DH##_r##ROWS##_any, DH, false, ROWS, false)       \
+  TA_FLASH_H16(ta_flash_attention_io16_dh##DH##_r##ROWS, DH, true, ROWS, true)               \
+  TA_FLASH_H16(ta_flash_attention_io16_dh##DH##_r##ROWS##_any, DH, true, ROWS, false)
+TA_FLASH_H16_FAMILY(64, 64)
+TA_FLASH_H16_FAMILY(64, 32)
+TA_FLASH_H16_FAMILY(128, 64)
+TA_FLASH_H16_FAMILY(128, 32)

@@ -308,7 +308,8 @@ typedef struct CopyArgs {
 // cache positions < min(kv_len, pos_base + i + 1) of kv head h /
 // group_size.  q/out element (h, i, d) sits at h * head_stride + i *
 // row_stride + d; kt is [H_kv, dh, t_max], v is [H_kv, t_max, dh].  The
-// grid is q_tiles * heads workgroups of 64 query rows.
+// grid is q_tiles * heads workgroups (ta_flash_rows / ta_flash16_rows query
+// rows each).
 typedef struct FlashArgs {
   const void *q;
   const void *kt;
@@ -420,14 +421,25 @@ typedef struct MlpArgs {
 #endif
 
 #ifdef __cplusplus
-// Work split of the causal prefill attention kernels, shared with the host
-// launch (threads = 64 * QB * KP, query tiles of 32 * QB rows).
+// Work split of the f32-cache causal prefill attention kernels, shared with
+// the host launch (threads = 64 * QB * KP, query tiles of 32 * QB rows).
 //   KP: key parts per query block (head dim 64: 4, head dim 128: 2)
 //   QB: 32-row query blocks per workgroup
 constexpr int ta_flash_parts(int dh) { return dh == 64 ? 4 : 2; }
 constexpr int ta_flash_qblocks(int /*dh*/) { return 2; }
 constexpr int ta_flash_threads(int dh) { return 64 * ta_flash_qblocks(dh) * ta_flash_parts(dh); }
 constexpr int ta_flash_rows(int dh) { return 32 * ta_flash_qblocks(dh); }
+
+// Query rows per workgroup (256 threads) of the f16-cache kernels: 32 while
+// all 32-row workgroups are on the chip at once (their LDS lets two share a
+// CU at head dim 64, one at 128), else 64.  Measured (us, 32 / 64 rows): 512
+// tokens x 32 heads, dh 64: 10.8 / 12.3; 128 tokens on a 1664-position cache,
+// 32 heads, dh 128: 32.1 / 42.0; 1024 tokens on 2048 positions, 16 heads, dh
+// 128 (512 workgroups of 32 rows): 50.2 / 42.3; 2048 tokens x 32 heads, dh
+// 64: 53.6 / 41.5.
+constexpr uint32_t ta_flash16_rows(uint32_t dh, uint32_t t_q, uint32_t heads, uint32_t cus) {
+  return (uint64_t)((t_q + 31u) / 32u) * heads <= (dh == 64 ? 2ull : 1ull) * cus ? 32u : 64u;
+}
 
 // Pipeline stages of the FP32-MFMA (_mi16) kernels: 8 for the 32-row
 // tiles (two waves per CU) and the 64 x 64 split-K tile (8 KiB stages), 4

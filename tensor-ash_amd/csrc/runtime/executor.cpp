@@ -2383,19 +2383,25 @@ ElemLaunch plan_flash(ExecutorImpl &e, const Tensor &q, const Tensor &kt, const 
   a.o_head_stride = o_hs;
   a.o_row_stride = o_rs;
   a.heads = heads;
-  const uint32_t rows = ta_flash_rows((int)dh); // query rows per workgroup
+  const uint32_t rows = kv16 ? ta_flash16_rows(dh, t_q, heads, e.ctx->cu_count())
+                             : (uint32_t)ta_flash_rows((int)dh); // query rows per workgroup
   a.q_tiles = (t_q + rows - 1) / rows;
   const uint64_t groups = (uint64_t)a.q_tiles * heads;
   if (groups == 0 || groups > UINT32_MAX)
     fail(op + ": empty or oversized launch (T_q " + std::to_string(t_q) + ", H " +
          std::to_string(heads) + ")");
-  const char *sym = io16 ? (dh == 64 ? "ta_flash_attention_io16_dh64"
-                                     : "ta_flash_attention_io16_dh128")
-                   : kv16 ? (dh == 64 ? "ta_flash_attention_kv16_dh64"
-                                      : "ta_flash_attention_kv16_dh128")
-                          : (dh == 64 ? "ta_flash_attention_dh64" : "ta_flash_attention_dh128");
-  ElemLaunch l = elem(sym, (uint32_t)groups, a);
-  l.threads = (uint32_t)ta_flash_threads((int)dh); // QB query blocks x KP key parts, 64 lanes each
+  std::string sym = "ta_flash_attention_";
+  if (kv16) {
+    // K rows of whole 16-byte pieces, within 32-bit offsets of a head's
+    // plane, are loaded straight into LDS.
+    const bool direct = t_max % 8 == 0 && t_max < (1u << 24);
+    sym += std::string(io16 ? "io16" : "kv16") + "_dh" + std::to_string(dh) + "_r" +
+           std::to_string(rows) + (direct ? "" : "_any");
+  } else {
+    sym += "dh" + std::to_string(dh);
+  }
+  ElemLaunch l = elem(sym.c_str(), (uint32_t)groups, a);
+  l.threads = kv16 ? 256u : (uint32_t)ta_flash_threads((int)dh);
   return l;
 }
 

@@ -230,3 +230,72 @@ def test_exec_ops_reject_before_launch(ta, ex):
     assert np.all(ex.download(b) == 3.0)
     with pytest.raises(ta.TensorAshError, match="empty"):
         ex.run_exec_ops([])
+
+
+# The f16-cache kernels at the edges of their tiles (32 / 64 query rows, 128
+# / 64 keys), with K rows of whole 16-byte pieces (T_max % 8 == 0) and
+# without, a prompt long enough for the 64-row tiles, and caches that end
+# inside a tile.  label, H, H_kv, T_q, T_max, dh, kv_len, pos_base, scale
+F16_CASES = [
+    ("one row, one key", 1, 1, 1, 1, 64, 1, 0, 0.125),
+    ("row tile minus one", 2, 1, 31, 40, 64, 31, 0, 0.125),
+    ("row tile plus one", 2, 2, 33, 33, 128, 33, 0, 0.09),
+    ("key tile plus one, odd cache", 4, 2, 65, 131, 64, 129, 64, 0.125),
+    ("key tile exact", 2, 1, 64, 128, 128, 128, 64, 0.09),
+    ("cache cut inside a tile", 2, 1, 130, 200, 64, 90, 20, 0.125),
+    ("64-row tiles", 32, 8, 600, 600, 64, 600, 0, 0.125),
+    ("64-row tiles, odd cache", 32, 4, 301, 333, 128, 311, 10, 0.09),
+    ("no valid position", 2, 2, 5, 16, 64, 0, 0, 0.125),
+    ("negative scale", 2, 2, 40, 64, 64, 40, 0, -0.125),
+    ("zero scale", 2, 2, 40, 64, 128, 40, 0, 0.0),
+]
+
+
+@pytest.mark.parametrize("io16", [False, True], ids=["kv16", "io16"])
+@pytest.mark.parametrize("label,heads,kv_heads,t_q,t_max,dh,kv_len,pos_base,scale", F16_CASES,
+                         ids=[c[0] for c in F16_CASES])
+def test_flash_f16_cache_tiles(ta, ex, oracle, label, heads, kv_heads, t_q, t_max, dh, kv_len, pos_base, scale, io16):
+    """Inputs in [-1, 1]: a score sums dh products with an error of at most
+    dh * 2^-24 = 7.6e-6, which bounds the weights' relative error; weights
+    and their sums add less, so 2e-5 absolute (|V| <= 1).  f16 results add
+    half an ulp of values up to 1 (2^-11).  Past kv_len the caches hold f16
+    infinities."""
+    q = oracle.fill_det(heads * t_q * dh, 5700)
+    if io16:
+        q = oracle.round_via_f16(q)
+    kt, v = fill_kv(oracle, kv_heads, dh, t_max, kv_len)
+    kt16, v16 = oracle.round_via_f16(kt), oracle.round_via_f16(v)
+    tq = ex.tensor_from(q, shape=[heads, t_q, dh], f16=io16)
+    tk = ex.tensor_from(kt, shape=[kv_heads, dh, t_max], f16=True)
+    tv = ex.tensor_from(v, shape=[kv_heads, t_max, dh], f16=True)
+    out = ex.tensor([heads, t_q, dh], f16=io16)
+    ex.flash_attention(tq, tk, tv, out, ta.FlashAttentionDesc(kv_len, pos_base, scale))
+    ref = oracle.flash_attention(q, kt16, v16, heads, kv_heads, t_q, t_max, dh, kv_len, pos_base, scale)
+    err, idx = oracle.max_abs_err(ex.download(out).reshape(-1), ref)
+    assert err <= 2e-5 + (2.0 ** -11 if io16 else 0.0), f"{label}: err {err} at {idx}"
+
+
+@pytest.mark.parametrize("io16", [False, True], ids=["kv16", "io16"])
+@pytest.mark.parametrize("dh,t_q", [(64, 70), (128, 70)])
+def test_flash_f16_cache_infinities(ta, ex, oracle, dh, t_q, io16):
+    """An infinite V entry makes that column infinite for the rows that
+    attend to it and leaves every other result finite; a key of -inf
+    (against positive q) has weight 0."""
+    heads = 2
+    q = oracle.round_via_f16(oracle.fill_det(heads * t_q * dh, 5800)).reshape(heads, t_q, dh)
+    q[:, :, 3] = np.abs(q[:, :, 3]) + np.float32(0.25)
+    kt, v = fill_kv(oracle, heads, dh, t_q, t_q)
+    kt, v = oracle.round_via_f16(kt).reshape(kt.shape), oracle.round_via_f16(v).reshape(v.shape)
+    kt[:, 3, 9] = -np.inf
+    v[0, 40, 5] = np.inf
+    out = ex.tensor([heads, t_q, dh], f16=io16)
+    ex.flash_attention(ex.tensor_from(q, f16=io16), ex.tensor_from(kt, f16=True), ex.tensor_from(v, f16=True), out,
+                       ta.FlashAttentionDesc(t_q, 0, 0.125))
+    got = ex.download(out)
+    safe = v.copy()
+    safe[0, 40, 5] = 0.0
+    ref = oracle.flash_attention(q, kt, safe, heads, heads, t_q, t_q, dh, t_q, 0, 0.125).reshape(got.shape)
+    hit = np.zeros(got.shape, bool)
+    hit[0, 40:, 5] = True
+    assert np.all(np.isposinf(got[hit]))
+    assert np.max(np.abs(got[~hit] - ref[~hit])) <= 2e-5 + (2.0 ** -11 if io16 else 0.0)
