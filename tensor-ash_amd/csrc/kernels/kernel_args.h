@@ -87,6 +87,43 @@ typedef struct GemmArgs {
   uint16_t *c16;
 } GemmArgs;
 
+// f32 product on bf16 matrix cores (ta_gemm_f32x6_*): every f32 operand is
+// written as three bf16 pieces in MFMA operand order by ta_pack_f32x3, and
+// six piece products are summed.  A packed operand is [plane][block of 32
+// rows (A) or columns (B)][k-step of 16][piece][lane][8 values]: 3 KiB per
+// block and k-step; blocks and k-steps past the matrix are zeros.
+#define TA_X6_STEP_BYTES 3072u
+// k-steps one workgroup of the pack covers (4 waves x 4 steps); it leaves
+// one word per row / column of its block: the OR of its values' bits.
+#define TA_X6_CHUNK_STEPS 16u
+
+typedef struct PackX3Job {
+  const float *src;
+  uint16_t *dst;
+  uint32_t *bits;  // [plane][chunk][blocks * 32]
+  uint64_t stride; // source elements between planes
+  uint32_t rows;   // A rows / B columns
+  uint32_t k;
+  uint32_t blocks, ksteps, chunks;
+  uint32_t groups; // workgroups of this job: planes * blocks (B: / 2) * chunks
+} PackX3Job;
+
+// Workgroups [0, a.groups) pack A ([rows, k], k contiguous), the rest B
+// ([k, rows], rows contiguous).
+typedef struct PackX3Args {
+  PackX3Job a, b;
+} PackX3Args;
+
+typedef struct GemmX6Args {
+  GemmArgs g; // the f32 operands and the fused epilogue (no split-K)
+  const uint16_t *pa;
+  const uint16_t *pb;
+  const uint32_t *bits_a;
+  const uint32_t *bits_b;
+  uint64_t plane_a, plane_b; // packed elements between planes (0 = broadcast)
+  uint32_t blocks_a, blocks_b, ksteps, chunks;
+} GemmX6Args;
+
 // Fixed-order reduction of split-K partial planes:
 // C[b][e] = sum_{s=0}^{S-1} scratch[(b * S + s) * mn + e].
 // The sum then takes the op's fused epilogue without alpha, which stage 1
@@ -451,6 +488,12 @@ constexpr uint32_t ta_flash16_rows(uint32_t dh, uint32_t t_q, uint32_t heads, ui
 constexpr int ta_mi16_stages(int bm, int bn) {
   return bm == 32 || (bm == 64 && bn == 64) ? TA_MI16_SKINNY_STAGES : 4;
 }
+
+// Threads of the ta_gemm_f32x6_<tile> kernels, and the waves' K groups (the
+// k-steps of a pipeline stage): 256 x 256 in 8 waves, 128 x 128 in 2 groups
+// of 4, 64 x 64 in 4 groups of 4.
+constexpr uint32_t ta_x6_threads(uint32_t tile) { return tile == 64 ? 1024u : 512u; }
+constexpr uint32_t ta_x6_groups(uint32_t tile) { return tile == 64 ? 4u : tile == 128 ? 2u : 1u; }
 
 // Threads of the pipelined f16-MFMA kernels (ta_gemm_{h16,a16}_<tile>_lds,
 // ta_gemm_h16sk_<tile>, ta_gemm_h16dual_<tile>_lds): 16 waves (four per

@@ -196,6 +196,9 @@ struct OpPlan {
   // 4 = covered, 5 = persistent GEMV-chain launch covering this op and the
   // next chain_jobs - 1, 6 = covered by it.
   int role = 0;
+  // Tile of the split-product form of an f32 GEMM (ta_gemm_f32x6_<tile>),
+  // 0 = the kernel's FP32-MFMA form.
+  uint32_t x6 = 0;
   uint32_t mlp_layers = 0;
   uint32_t chain_jobs = 0;
 };
@@ -327,6 +330,32 @@ struct ExecutorImpl {
     return plan;
   }
 
+  // The heuristic's pick may run in its split-product form; an explicit
+  // kernel selection, or a tuned kernel or split count that differs from
+  // the heuristic's, runs as named.
+  void choose_x6(const ResolvedMatmul &d, OpPlan &plan) const {
+    if (!selection.is_auto() || d.a_f16 || d.b_f16 || d.packed_b)
+      return;
+    const uint32_t cus = ctx->cu_count();
+    const size_t heur = heuristic_kernel_index(cus, d.batch, d.m, d.n, d.k, false, false);
+    if (auto e = tuned_entry(TuneKey{d.batch, d.m, d.n, d.k, false}))
+      if (e->kernel != heur || e->splitk2_splits)
+        return;
+    // TA_F32X6 fixes the form (route control): 0, or the tile.
+    if (const char *env = std::getenv("TA_F32X6")) {
+      const uint32_t tile = (uint32_t)std::strtoul(env, nullptr, 10);
+      const bool ok = (tile == 64 || tile == 128 || tile == 256) && !KERNEL_SPECS[heur].is_gemv() &&
+                      f32x6_plan(d, tile).bytes <= kF32X6ScratchCapBytes;
+      plan.x6 = ok ? tile : 0;
+    } else {
+      plan.x6 = f32x6_tile(cus, d, KERNEL_SPECS[plan.splitk2 ? plan.kernel : heur], plan.splitk2);
+    }
+    if (plan.x6) {
+      plan.splitk2.reset();
+      plan.kernel = heur;
+    }
+  }
+
   // Auto routes whose kernel cannot honour an op's decode fusions fall
   // back onto the heuristic pick when that one can (src/executor/mod.rs:
   // 259-315, demote_for_op); explicit selections keep their loud failure
@@ -363,7 +392,9 @@ struct ExecutorImpl {
         p.kernel = *selection.index;
       return p;
     }
-    return plan_shape(d.batch, d.m, d.n, d.k, d.b_f16, splitk_eligible);
+    OpPlan p = plan_shape(d.batch, d.m, d.n, d.k, d.b_f16, splitk_eligible);
+    choose_x6(d, p);
+    return p;
   }
 
   // ---- launches ----
@@ -378,7 +409,9 @@ struct ExecutorImpl {
   ScratchNeed scratch_need(const ResolvedMatmul &d, const OpPlan &p) const {
     ScratchNeed need;
     const KernelSpec &s = KERNEL_SPECS[p.kernel];
-    if (p.splitk2) {
+    if (p.x6) {
+      need.splitk = f32x6_plan(d, p.x6).bytes;
+    } else if (p.splitk2) {
       need.splitk = (uint64_t)d.batch * d.m * d.n * *p.splitk2 *
                     splitk_sub_splits(ctx->cu_count(), d, *p.splitk2) * 4;
     } else if (s.is_gemv()) {
@@ -482,7 +515,8 @@ struct ExecutorImpl {
   // region and entered in the cache, where the ops then find them: one
   // launch instead of two on the submission's critical path (the prefill
   // layer converts x for QKV and up/gate and the attention output for O).
-  // Not with split-K ops in the submission: their planes share the region.
+  // Not with split-K or split-product ops in the submission: their planes
+  // and packed operands share the region.
   void convert_inputs_up_front(const std::vector<MatmulOp> &ops,
                                const std::vector<ResolvedMatmul> &res,
                                const std::vector<OpPlan> &plans, Scratch &scratch, CvtCache &cvt,
@@ -490,7 +524,7 @@ struct ExecutorImpl {
     if (std::getenv("TA_NO_CVT_PAIR"))
       return;
     for (const auto &p : plans)
-      if (p.splitk2)
+      if (p.splitk2 || p.x6)
         return;
     std::vector<CvtCandidate> cand(ops.size());
     for (size_t i = 0; i < ops.size(); ++i) {
@@ -552,11 +586,56 @@ struct ExecutorImpl {
            a_elems == (uint64_t)res[i].batch * res[i].m * res[i].n;
   }
 
+  // Split-product form of an f32 GEMM: pack both operands, then multiply.
+  void launch_x6(const ResolvedMatmul &d, GemmArgs &a, uint32_t tile, Scratch &scratch,
+                 hipStream_t stream) const {
+    const F32X6Plan x = f32x6_plan(d, tile);
+    if (scratch.splitk_bytes < x.bytes)
+      fail("internal: packed operand scratch not reserved");
+    char *base = static_cast<char *>(scratch.splitk);
+    auto job = [&](const void *src, uint64_t off, uint64_t bits_off, uint64_t stride, uint32_t rows,
+                   uint32_t blocks, uint32_t wide, uint64_t planes) {
+      PackX3Job j{};
+      j.src = static_cast<const float *>(src);
+      j.dst = reinterpret_cast<uint16_t *>(base + off);
+      j.bits = reinterpret_cast<uint32_t *>(base + bits_off);
+      j.stride = stride;
+      j.rows = rows;
+      j.k = d.k;
+      j.blocks = blocks;
+      j.ksteps = x.ksteps;
+      j.chunks = x.chunks;
+      j.groups = (uint32_t)(planes * (blocks / wide) * x.chunks);
+      return j;
+    };
+    PackX3Args pk{};
+    pk.a = job(a.a, 0, x.bits_a_off, d.batch_stride_a, d.m, x.blocks_a, 1, x.planes_a);
+    pk.b = job(a.b, x.b_off, x.bits_b_off, d.batch_stride_b, d.n, x.blocks_b, 2, x.planes_b);
+    launch("ta_pack_f32x3", pk.a.groups + pk.b.groups, 1, 1, 256, &pk, stream);
+    GemmX6Args g{};
+    a.tiles_m = div_ceil(d.m, tile);
+    a.tiles_n = div_ceil(d.n, tile);
+    g.g = a;
+    g.pa = pk.a.dst;
+    g.pb = pk.b.dst;
+    g.bits_a = pk.a.bits;
+    g.bits_b = pk.b.bits;
+    g.plane_a = d.batch_stride_a ? (uint64_t)x.blocks_a * x.ksteps * (TA_X6_STEP_BYTES / 2) : 0;
+    g.plane_b = d.batch_stride_b ? (uint64_t)x.blocks_b * x.ksteps * (TA_X6_STEP_BYTES / 2) : 0;
+    g.blocks_a = x.blocks_a;
+    g.blocks_b = x.blocks_b;
+    g.ksteps = x.ksteps;
+    g.chunks = x.chunks;
+    const std::string t = std::to_string(tile);
+    launch("ta_gemm_f32x6_m" + t + "n" + t, a.tiles_m * a.tiles_n, 1, d.batch, ta_x6_threads(tile), &g,
+           stream);
+  }
+
   // `up` set: dual SwiGLU launch (ta_gemm_h16dual_*) computing `up`
   // (plain) and `op` (gate with activation and Mul{d = up.C}) in one pass.
   void launch_gemm(const KernelSpec &s, const ResolvedMatmul &d, const MatmulOp &op,
                    uint32_t splits, Scratch &scratch, CvtCache &cvt, hipStream_t stream,
-                   const MatmulOp *up = nullptr, uint16_t *c16 = nullptr) const {
+                   const MatmulOp *up = nullptr, uint16_t *c16 = nullptr, uint32_t x6 = 0) const {
     void *splitk_scratch = scratch.splitk;
     GemmArgs a{};
     a.a = op.call.a->device_ptr();
@@ -585,6 +664,11 @@ struct ExecutorImpl {
       if (const Tensor *dt = op.epilogue.d_tensor())
         a.d = static_cast<const float *>(dt->device_ptr());
       a.beta = op.epilogue.binary.beta;
+    }
+    if (x6) {
+      cvt.drop_region(); // the packed operands overwrite the f16 copies
+      launch_x6(d, a, x6, scratch, stream);
+      return;
     }
     a.tiles_m = div_ceil(d.m, s.tile_m);
     a.tiles_n = div_ceil(d.n, s.tile_n);
@@ -1330,7 +1414,7 @@ struct ExecutorImpl {
                                        (uint64_t)res[i].batch * res[i].m * res[i].n, c16, i, -1});
       } else
         launch_gemm(s, res[i], ops[i], p.splitk2.value_or(1), scratch, cvt, stream,
-                    p.role == 2 ? &ops[i - 1] : nullptr);
+                    p.role == 2 ? &ops[i - 1] : nullptr, nullptr, p.x6);
     }
   }
 
@@ -1785,7 +1869,7 @@ struct ExecutorImpl {
     for (size_t i = 0; i < res.size(); ++i) {
       const ResolvedMatmul &d = res[i];
       const KernelSpec &s = KERNEL_SPECS[plans[i].kernel];
-      if (plans[i].splitk2 || s.is_gemv())
+      if (plans[i].splitk2 || plans[i].x6 || s.is_gemv())
         continue;
       const double tiles = (double)d.batch * div_ceil(d.m, s.tile_m) * div_ceil(d.n, s.tile_n);
       if (tiles >= cus / 2)
@@ -1842,8 +1926,13 @@ struct ExecutorImpl {
   // for f32 operands.  The allocating and the allocation-free entry
   // points share it, so they launch the same kernels.
   OpPlan split_k2_plan(const MatmulOp &op, const ResolvedMatmul &d, uint32_t splits) const {
-    if (splits <= 1)
-      return plan_op(op, d, false);
+    if (splits <= 1) {
+      // on the FP32 MFMAs: the allocation-free form has no room for packed
+      // operands, and both forms give the same bits
+      OpPlan p = plan_op(op, d, false);
+      p.x6 = 0;
+      return p;
+    }
     OpPlan p;
     p.kernel = registry_index(splitk_stage1_spec(d.m, d.n, d.k).name);
     p.splitk2 = splits;
@@ -2883,6 +2972,16 @@ DispatchInfo Executor::dispatch_info(uint32_t batch, uint32_t m, uint32_t n, uin
 DispatchInfo Executor::dispatch_info_for(uint32_t batch, uint32_t m, uint32_t n, uint32_t k,
                                          bool b_f16) const {
   OpPlan p = impl_->plan_shape(batch, m, n, k, b_f16, true);
+  if (!b_f16) {
+    ResolvedMatmul d;
+    d.batch = batch;
+    d.m = m;
+    d.n = n;
+    d.k = k;
+    d.batch_stride_a = d.batch_stride_b = batch > 1 ? 1 : 0;
+    d.total_flops = 2ull * batch * m * n * k;
+    impl_->choose_x6(d, p);
+  }
   const KernelSpec &s = p.splitk2 ? splitk_stage1_spec(m, n, k) : KERNEL_SPECS[p.kernel];
   DispatchInfo info;
   info.kernel = s.name;

@@ -93,6 +93,21 @@ void validate_scratch_geometry(uint32_t batch, uint32_t m, uint32_t n, uint32_t 
 std::optional<uint64_t> checked_auto_scratch_end(uint64_t offset, uint64_t bytes);
 
 // ---- GEMV geometry ----
+// Layout of one f32 op on the split-product route (ta_pack_f32x3 +
+// ta_gemm_f32x6_<tile>): packed A, packed B, then their row / column bits,
+// in one scratch region of `bytes`.
+struct F32X6Plan {
+  uint32_t blocks_a, blocks_b, ksteps, chunks;
+  uint64_t planes_a, planes_b;
+  uint64_t b_off, bits_a_off, bits_b_off, bytes;
+};
+F32X6Plan f32x6_plan(const ResolvedMatmul &dims, uint32_t tile);
+// Tile (256, 128, 64) of the split-product route when it is the faster one
+// for this shape, else 0.  `fp32`, `splits`: the route it would replace.
+uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &dims, const KernelSpec &fp32,
+                    std::optional<uint32_t> splits);
+constexpr uint64_t kF32X6ScratchCapBytes = 1ull << 30;
+
 struct GemvPlan {
   uint32_t tw = 64, mr = 1, tiles = 0, kchunk = 0, kchunks = 1;
   uint64_t partial_bytes = 0; // 0 when kchunks == 1

@@ -2,6 +2,7 @@
 // GEMV geometry, and the pure helpers of the measured tuner.
 #include <algorithm>
 #include <cctype>
+#include <cmath>
 #include <cstdlib>
 #include <sstream>
 
@@ -394,6 +395,70 @@ uint32_t default_num_k_splits(uint32_t cus, uint32_t batch, uint32_t m, uint32_t
   const uint64_t raw = std::max<uint64_t>(1, (2ull * cus + tiles - 1) / tiles);
   const uint64_t max_splits = std::max<uint64_t>(1, k / 32);
   return (uint32_t)std::min<uint64_t>({raw, max_splits, 0xFFFF});
+}
+
+// ---- f32 products on the bf16 matrix cores ----
+F32X6Plan f32x6_plan(const ResolvedMatmul &d, uint32_t tile) {
+  F32X6Plan p{};
+  const uint32_t g = ta_x6_groups(tile);
+  p.blocks_a = div_ceil(d.m, tile) * (tile / 32);
+  p.blocks_b = div_ceil(d.n, tile) * (tile / 32);
+  p.ksteps = div_ceil(div_ceil(d.k, 16), g) * g;
+  p.chunks = div_ceil(p.ksteps, TA_X6_CHUNK_STEPS);
+  p.planes_a = d.batch_stride_a ? d.batch : 1;
+  p.planes_b = d.batch_stride_b ? d.batch : 1;
+  p.b_off = p.planes_a * p.blocks_a * p.ksteps * TA_X6_STEP_BYTES;
+  p.bits_a_off = p.b_off + p.planes_b * p.blocks_b * p.ksteps * TA_X6_STEP_BYTES;
+  p.bits_b_off = p.bits_a_off + p.planes_a * p.chunks * p.blocks_a * 32 * 4;
+  p.bytes = p.bits_b_off + p.planes_b * p.chunks * p.blocks_b * 32 * 4;
+  return p;
+}
+
+// Both sides are estimated from measured rates (us, 256 CUs).
+// Split products: the pack (one launch: 6.5 us, 10 B per element at 5.5
+// TB/s), the gap to the GEMM and its ramp, then rounds of tiles, each k-step
+// (16) of a round at 2.2 us (256 x 256), 0.6 (128 x 128, two K groups) or
+// 0.21 (64 x 64, four): 4096^3 561 us on 256 tiles, 3000^3 331 us and
+// 2048^3 93 us on 128 x 128, 512x2048x2048 30 us on 64 x 64.
+// FP32 MFMA: 3.6 us per k-step and round for whole 256 x 256 tiles, 2.0 /
+// 1.4 / 0.8 / 0.52 for the smaller ones; tiles that cross the matrix's edge
+// load scalars, and the launch waits for them (3000^3 on 256 x 128: 6.4 us;
+// 1000x1531x777 on 64 x 64: 1.0).  Split-K: 75 TFLOP/s plus 10 us.
+uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &fp32,
+                    std::optional<uint32_t> splits) {
+  if (d.a_f16 || d.b_f16 || d.packed_b || fp32.kind != KernelKind::GemmF32 || d.batch > 65535 ||
+      d.m < 32 || d.n < 32 || d.k < 64)
+    return 0;
+  const double ksteps = (d.k + 15) / 16;
+  double old_us;
+  if (splits) {
+    old_us = 10.0 + (double)d.total_flops / 75e6;
+  } else {
+    const bool whole = d.m % fp32.tile_m == 0 && d.n % fp32.tile_n == 0;
+    const uint32_t area = fp32.tile_m * fp32.tile_n;
+    const double step = area >= 256 * 256   ? (whole ? 3.6 : 9.0)
+                        : area >= 256 * 128 ? (whole ? 2.0 : 6.4)
+                        : area >= 128 * 128 ? (whole ? 1.4 : 3.2)
+                        : area >= 128 * 64  ? (whole ? 0.8 : 1.8)
+                                            : (whole ? 0.52 : 1.0);
+    const double tiles = (double)d.batch * div_ceil(d.m, fp32.tile_m) * div_ceil(d.n, fp32.tile_n);
+    const double rounds = area >= 128 * 128 ? std::ceil(tiles / cus) : std::max(1.0, tiles / cus);
+    old_us = 3.0 + rounds * ksteps * step;
+  }
+  const double planes_a = d.batch_stride_a ? d.batch : 1, planes_b = d.batch_stride_b ? d.batch : 1;
+  const double pack_us =
+      6.5 + 10.0 * d.k * (planes_a * (double)d.m + planes_b * (double)d.n) / 5.5e6;
+  uint32_t best = 0;
+  double best_us = 0.95 * old_us;
+  for (const auto &[tile, step] : {std::pair<uint32_t, double>{256, 2.2}, {128, 0.6}, {64, 0.21}}) {
+    const double tiles = (double)d.batch * div_ceil(d.m, tile) * div_ceil(d.n, tile);
+    const double us = pack_us + 5.0 + std::ceil(tiles / cus) * ksteps * step;
+    if (us < best_us && f32x6_plan(d, tile).bytes <= kF32X6ScratchCapBytes) {
+      best_us = us;
+      best = tile;
+    }
+  }
+  return best;
 }
 
 // splitk2.rs:226-246.

@@ -1,0 +1,107 @@
+"""The split-product form of f32 GEMMs (three bf16 pieces per value, six
+piece products): sizes at the edges of its tiles, K steps and pack chunks,
+every epilogue operand, batches with and without broadcast, its accuracy
+beside the FP32-MFMA form, and the values it hands to that form."""
+
+import numpy as np
+import pytest
+
+from test_gemm_gpu import check_f32, run_case
+
+pytestmark = pytest.mark.gpu
+
+TILES = [64, 128, 256]
+
+
+def rel2(got, exact):
+    return float(np.linalg.norm(got.astype(np.float64) - exact) / np.linalg.norm(exact))
+
+
+def product(ta, ex, a, b, monkeypatch, form):
+    monkeypatch.setenv("TA_F32X6", str(form))
+    ta_, tb = ex.tensor_from(a), ex.tensor_from(b)
+    c = ex.tensor([a.shape[0], b.shape[1]])
+    ex.run_ops([ta.MatmulOp(ta_, tb, c)])
+    return ex.download(c)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k", [(9, 1, 1), (64, 64, 16), (65, 63, 17), (129, 127, 255), (256, 256, 256),
+                                   (257, 255, 257), (300, 520, 1000)])
+def test_x6_tile_edges(ta, ex, oracle, monkeypatch, tile, m, n, k):
+    monkeypatch.setenv("TA_F32X6", str(tile))
+    run_case(ta, ex, oracle, m, n, k)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("epi", [dict(bias=[257], act=1), dict(bias=[257], act=3), dict(act=2, binary=2),
+                                 dict(binary=1, beta=0.5, alpha=0.75, accumulate=True)])
+def test_x6_epilogues(ta, ex, oracle, monkeypatch, tile, epi):
+    monkeypatch.setenv("TA_F32X6", str(tile))
+    run_case(ta, ex, oracle, 130, 257, 129, **epi)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("ba,bb,bc", [(3, 1, 3), (1, 3, 3), (3, 3, 3)])
+def test_x6_batches(ta, ex, oracle, monkeypatch, tile, ba, bb, bc):
+    monkeypatch.setenv("TA_F32X6", str(tile))
+    run_case(ta, ex, oracle, 70, 90, 300, batch_a=ba, batch_b=bb, batch_c=bc)
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 520, 777), (512, 2048, 2048)])
+def test_x6_error_is_no_larger_than_the_fp32_form(ta, ex, monkeypatch, m, n, k):
+    """Against f64, normal inputs: at most the data-parallel FP32-MFMA
+    form's error (a tenth allowed for the draw)."""
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    errs = {form: rel2(product(ta, ex, a, b, monkeypatch, form), exact) for form in [0] + TILES}
+    print(errs, flush=True)
+    for tile in TILES:
+        assert errs[tile] <= 1.1 * errs[0], errs
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_x6_special_values(ta, ex, monkeypatch, tile):
+    """Infinities, NaN, values next to the largest f32 and rows of tiny
+    values give what f32 arithmetic gives."""
+    rng = np.random.default_rng(7)
+    m, n, k = 200, 150, 96
+    a, b = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32), rng.uniform(0.5, 1.5, (k, n)).astype(np.float32)
+    a[3, 5], a[70, 1], a[150, 9] = np.inf, np.nan, np.float32(3.402e38)
+    a[100] *= np.float32(2.0 ** -112)  # every value below 2^-95
+    b[7, 33] = -np.inf
+    got = product(ta, ex, a, b, monkeypatch, tile)
+    with np.errstate(all="ignore"):
+        exact = a.astype(np.float64) @ b.astype(np.float64)
+    # the row past the largest f32 meets the column with -inf: +inf - inf in
+    # f32, in an order of its own
+    got[150, 33] = exact[150, 33]
+    assert np.argwhere(np.isnan(got) != np.isnan(exact)).tolist() == []
+    inf = np.isinf(exact)
+    assert np.array_equal(got[inf], exact[inf].astype(np.float32))
+    # row 150 sums past the largest f32 where its big value meets b > 1
+    fine = np.isfinite(exact) & (np.abs(exact) < 3.2e38)
+    big = np.isfinite(exact) & (np.abs(exact) > 3.5e38)
+    assert np.all(np.isposinf(got[big])) and np.any(big)
+    assert np.max(np.abs(got[fine] - exact[fine]) / np.abs(exact[fine])) <= 2 * k * 2.0 ** -24
+
+
+def test_x6_in_graphs_and_prepared(ta, ex, oracle, monkeypatch):
+    """A dependent graph of two products, run and prepared (replayed): the
+    bits of the products submitted alone."""
+    monkeypatch.setenv("TA_F32X6", "128")
+    m, k = 150, 200
+    a, b, d = (oracle.fill_det(m * k, 1), oracle.fill_det(k * k, 2), oracle.fill_det(k * k, 3))
+    x, w1, w2 = ex.tensor_from(a, shape=[m, k]), ex.tensor_from(b, shape=[k, k]), ex.tensor_from(d, shape=[k, k])
+    y, z = ex.tensor([m, k]), ex.tensor([m, k])
+    ops = [ta.MatmulOp(x, w1, y), ta.MatmulOp(y, w2, z, epilogue=ta.Epilogue(activation=ta.ACTIVATION_RELU))]
+    for op in ops:
+        ex.run_ops([op])
+    alone = ex.download(z)
+    check_f32(ex.download(y).reshape(-1), oracle.reference_gemm(a, b, 1, m, k, k), k, oracle)
+    prep = ex.prepare_op_graph(ops)
+    for run in (lambda: ex.run_op_graph(ops), prep.run, prep.run):
+        ex.upload(z, np.zeros((m, k), np.float32))
+        run()
+        assert np.array_equal(ex.download(z), alone)
