@@ -124,6 +124,21 @@ typedef struct GemmX6Args {
   uint32_t blocks_a, blocks_b, ksteps, chunks;
 } GemmX6Args;
 
+// Few rows of f32 A on f16 weights (ta_gemm_f16w3_*): A packed by
+// ta_pack_f32x3 (blocks of 32 rows, K padded to whole stages), B as it lies
+// in memory.  gridDim.y workgroups share each output tile's K stages and
+// meet as the in-kernel split-K GEMMs do (g.partial, g.counters, g.k_splits).
+#define TA_W3_BN 64u
+#define TA_W3_BK 64u
+typedef struct GemmW3Args {
+  GemmArgs g;
+  const uint16_t *pa;
+  const uint32_t *bits_a;
+  uint64_t plane_a; // packed elements between planes (0 = broadcast)
+  uint32_t blocks_a, ksteps, chunks;
+  uint32_t pad;
+} GemmW3Args;
+
 // Fixed-order reduction of split-K partial planes:
 // C[b][e] = sum_{s=0}^{S-1} scratch[(b * S + s) * mn + e].
 // The sum then takes the op's fused epilogue without alpha, which stage 1

@@ -199,6 +199,8 @@ struct OpPlan {
   // Tile of the split-product form of an f32 GEMM (ta_gemm_f32x6_<tile>),
   // 0 = the kernel's FP32-MFMA form.
   uint32_t x6 = 0;
+  // Few rows on f16 weights: the split-product kernel (ta_gemm_f16w3_*).
+  bool w3 = false;
   uint32_t mlp_layers = 0;
   uint32_t chain_jobs = 0;
 };
@@ -394,6 +396,10 @@ struct ExecutorImpl {
     }
     OpPlan p = plan_shape(d.batch, d.m, d.n, d.k, d.b_f16, splitk_eligible);
     choose_x6(d, p);
+    // The heuristic's pick for few rows (as above, not a named or tuned one).
+    p.w3 = selection.is_auto() && KERNEL_SPECS[p.kernel].kind == KernelKind::GemmF16w && w3_ok(d) &&
+           !std::getenv("TA_NO_W3") &&
+           p.kernel == heuristic_kernel_index(ctx->cu_count(), d.batch, d.m, d.n, d.k, true, false);
     return p;
   }
 
@@ -411,6 +417,11 @@ struct ExecutorImpl {
     const KernelSpec &s = KERNEL_SPECS[p.kernel];
     if (p.x6) {
       need.splitk = f32x6_plan(d, p.x6).bytes;
+    } else if (p.w3) {
+      const W3Plan w = w3_plan(ctx->cu_count(), d);
+      need.splitk = 2 * w.pack_bytes; // two packed A's (CvtCache)
+      need.partial = w.partial_bytes;
+      need.counters = w.counters;
     } else if (p.splitk2) {
       need.splitk = (uint64_t)d.batch * d.m * d.n * *p.splitk2 *
                     splitk_sub_splits(ctx->cu_count(), d, *p.splitk2) * 4;
@@ -457,14 +468,15 @@ struct ExecutorImpl {
     void *base = nullptr;       // where the copy lives
     size_t producer = SIZE_MAX; // op whose epilogue wrote it, if any
     int half = -1;              // split-K region half, -1 = elsewhere
+    uint32_t packed_k = 0;      // f16 copy: 0; packed pieces (ta_pack_f32x3): their K
     uint64_t age = 0;
   };
   struct CvtCache {
     CvtEntry e[2];
     uint64_t clock = 0;
-    CvtEntry *find(const void *buffer, const void *src, uint64_t n) {
+    CvtEntry *find(const void *buffer, const void *src, uint64_t n, uint32_t packed_k = 0) {
       for (auto &x : e)
-        if (x.buffer && x.buffer == buffer && x.src == src && x.n == n)
+        if (x.buffer && x.buffer == buffer && x.src == src && x.n == n && x.packed_k == packed_k)
           return &x;
       return nullptr;
     }
@@ -586,6 +598,70 @@ struct ExecutorImpl {
            a_elems == (uint64_t)res[i].batch * res[i].m * res[i].n;
   }
 
+  static PackX3Job pack_job(const void *src, char *dst, char *bits, uint64_t stride, uint32_t rows,
+                            uint32_t k, uint32_t blocks, uint32_t ksteps, uint32_t chunks,
+                            uint32_t wide, uint64_t planes) {
+    PackX3Job j{};
+    j.src = static_cast<const float *>(src);
+    j.dst = reinterpret_cast<uint16_t *>(dst);
+    j.bits = reinterpret_cast<uint32_t *>(bits);
+    j.stride = stride;
+    j.rows = rows;
+    j.k = k;
+    j.blocks = blocks;
+    j.ksteps = ksteps;
+    j.chunks = chunks;
+    j.groups = (uint32_t)(planes * (blocks / wide) * chunks);
+    return j;
+  }
+
+  // Few rows of f32 A on f16 weights: pack A (once per distinct A of a
+  // submission, kept like the f16 copies), then multiply.
+  void launch_w3(const ResolvedMatmul &d, const MatmulOp &op, GemmArgs &a, Scratch &scratch,
+                 CvtCache &cvt, hipStream_t stream) const {
+    const W3Plan w = w3_plan(ctx->cu_count(), d);
+    if (scratch.partial_bytes < w.partial_bytes || scratch.counters_len < w.counters)
+      fail("internal: split-product scratch not reserved");
+    const void *buf = op.call.a->buffer_id();
+    // rows x K of one plane, its planes and its padding decide the layout
+    const uint64_t n = w.planes * d.m * d.k;
+    char *packed = nullptr;
+    if (CvtEntry *hit = cvt.find(buf, a.a, n, d.k)) {
+      packed = static_cast<char *>(hit->base);
+    } else {
+      CvtEntry &v = cvt.victim();
+      const CvtEntry &other = &v == &cvt.e[0] ? cvt.e[1] : cvt.e[0];
+      const int half = other.half == 0 ? 1 : 0;
+      const uint64_t half_bytes = scratch.splitk_bytes / 2 / 256 * 256;
+      if (w.pack_bytes > half_bytes)
+        fail("internal: packed operand scratch not reserved");
+      packed = static_cast<char *>(scratch.splitk) + half * half_bytes;
+      PackX3Args pk{};
+      pk.a = pack_job(a.a, packed, packed + w.bits_off, d.batch_stride_a, d.m, d.k, w.blocks, w.ksteps,
+                      w.chunks, 1, w.planes);
+      launch("ta_pack_f32x3", pk.a.groups, 1, 1, 256, &pk, stream);
+      CvtEntry e{buf, a.a, n, packed, SIZE_MAX, half};
+      e.packed_k = d.k;
+      cvt.put(v, e);
+    }
+    GemmW3Args g{};
+    a.tiles_m = w.tiles_m;
+    a.tiles_n = w.tiles_n;
+    a.k_splits = w.splits;
+    a.partial = static_cast<float *>(scratch.partial);
+    a.counters = scratch.counters;
+    g.g = a;
+    g.pa = reinterpret_cast<uint16_t *>(packed);
+    g.bits_a = reinterpret_cast<uint32_t *>(packed + w.bits_off);
+    g.plane_a = d.batch_stride_a ? (uint64_t)w.blocks * w.ksteps * (TA_X6_STEP_BYTES / 2) : 0;
+    g.blocks_a = w.blocks;
+    g.ksteps = w.ksteps;
+    g.chunks = w.chunks;
+    // whole 16-byte pieces of B's rows go straight to LDS
+    launch("ta_gemm_f16w3_r" + std::to_string(w.rows) + (d.n % 8 == 0 ? "" : "_any"),
+           w.tiles_m * w.tiles_n, w.splits, d.batch, 512, &g, stream);
+  }
+
   // Split-product form of an f32 GEMM: pack both operands, then multiply.
   void launch_x6(const ResolvedMatmul &d, GemmArgs &a, uint32_t tile, Scratch &scratch,
                  hipStream_t stream) const {
@@ -593,24 +669,11 @@ struct ExecutorImpl {
     if (scratch.splitk_bytes < x.bytes)
       fail("internal: packed operand scratch not reserved");
     char *base = static_cast<char *>(scratch.splitk);
-    auto job = [&](const void *src, uint64_t off, uint64_t bits_off, uint64_t stride, uint32_t rows,
-                   uint32_t blocks, uint32_t wide, uint64_t planes) {
-      PackX3Job j{};
-      j.src = static_cast<const float *>(src);
-      j.dst = reinterpret_cast<uint16_t *>(base + off);
-      j.bits = reinterpret_cast<uint32_t *>(base + bits_off);
-      j.stride = stride;
-      j.rows = rows;
-      j.k = d.k;
-      j.blocks = blocks;
-      j.ksteps = x.ksteps;
-      j.chunks = x.chunks;
-      j.groups = (uint32_t)(planes * (blocks / wide) * x.chunks);
-      return j;
-    };
     PackX3Args pk{};
-    pk.a = job(a.a, 0, x.bits_a_off, d.batch_stride_a, d.m, x.blocks_a, 1, x.planes_a);
-    pk.b = job(a.b, x.b_off, x.bits_b_off, d.batch_stride_b, d.n, x.blocks_b, 2, x.planes_b);
+    pk.a = pack_job(a.a, base, base + x.bits_a_off, d.batch_stride_a, d.m, d.k, x.blocks_a, x.ksteps,
+                    x.chunks, 1, x.planes_a);
+    pk.b = pack_job(a.b, base + x.b_off, base + x.bits_b_off, d.batch_stride_b, d.n, d.k, x.blocks_b,
+                    x.ksteps, x.chunks, 2, x.planes_b);
     launch("ta_pack_f32x3", pk.a.groups + pk.b.groups, 1, 1, 256, &pk, stream);
     GemmX6Args g{};
     a.tiles_m = div_ceil(d.m, tile);
@@ -635,7 +698,8 @@ struct ExecutorImpl {
   // (plain) and `op` (gate with activation and Mul{d = up.C}) in one pass.
   void launch_gemm(const KernelSpec &s, const ResolvedMatmul &d, const MatmulOp &op,
                    uint32_t splits, Scratch &scratch, CvtCache &cvt, hipStream_t stream,
-                   const MatmulOp *up = nullptr, uint16_t *c16 = nullptr, uint32_t x6 = 0) const {
+                   const MatmulOp *up = nullptr, uint16_t *c16 = nullptr, uint32_t x6 = 0,
+                   bool w3 = false) const {
     void *splitk_scratch = scratch.splitk;
     GemmArgs a{};
     a.a = op.call.a->device_ptr();
@@ -668,6 +732,10 @@ struct ExecutorImpl {
     if (x6) {
       cvt.drop_region(); // the packed operands overwrite the f16 copies
       launch_x6(d, a, x6, scratch, stream);
+      return;
+    }
+    if (w3) {
+      launch_w3(d, op, a, scratch, cvt, stream);
       return;
     }
     a.tiles_m = div_ceil(d.m, s.tile_m);
@@ -1414,7 +1482,7 @@ struct ExecutorImpl {
                                        (uint64_t)res[i].batch * res[i].m * res[i].n, c16, i, -1});
       } else
         launch_gemm(s, res[i], ops[i], p.splitk2.value_or(1), scratch, cvt, stream,
-                    p.role == 2 ? &ops[i - 1] : nullptr, nullptr, p.x6);
+                    p.role == 2 ? &ops[i - 1] : nullptr, nullptr, p.x6, p.w3);
     }
   }
 
@@ -1869,7 +1937,7 @@ struct ExecutorImpl {
     for (size_t i = 0; i < res.size(); ++i) {
       const ResolvedMatmul &d = res[i];
       const KernelSpec &s = KERNEL_SPECS[plans[i].kernel];
-      if (plans[i].splitk2 || plans[i].x6 || s.is_gemv())
+      if (plans[i].splitk2 || plans[i].x6 || plans[i].w3 || s.is_gemv())
         continue;
       const double tiles = (double)d.batch * div_ceil(d.m, s.tile_m) * div_ceil(d.n, s.tile_n);
       if (tiles >= cus / 2)

@@ -108,6 +108,17 @@ uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &dims, const KernelSpec &
                     std::optional<uint32_t> splits);
 constexpr uint64_t kF32X6ScratchCapBytes = 1ull << 30;
 
+// An op of few rows on f16 weights on the split-product route
+// (ta_gemm_f16w3_r<rows>): packed A, K splits and scratch.
+struct W3Plan {
+  uint32_t rows; // 32 or 64 per workgroup
+  uint32_t blocks, ksteps, chunks, tiles_m, tiles_n, splits;
+  uint64_t planes, bits_off, pack_bytes;
+  uint64_t partial_bytes, counters;
+};
+W3Plan w3_plan(uint32_t cus, const ResolvedMatmul &dims);
+bool w3_ok(const ResolvedMatmul &dims);
+
 struct GemvPlan {
   uint32_t tw = 64, mr = 1, tiles = 0, kchunk = 0, kchunks = 1;
   uint64_t partial_bytes = 0; // 0 when kchunks == 1

@@ -461,6 +461,38 @@ uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &fp3
   return best;
 }
 
+// ---- few rows on f16 weights ----
+// Up to 64 rows that are no decode GEMV (9 to 64 rows, or fewer in a batch).
+// With more rows and at least 64 columns the f16-MFMA route rounds A.  Below
+// 160 rows of K the pack's launch costs more than it saves (us, split / FP32
+// MFMA: K = 110, 33 x 5007: 16.4 / 14.6; K = 64: 10.7 / 9.0; K = 500, 40 x
+// 300: 25 / 39).
+bool w3_ok(const ResolvedMatmul &d) {
+  return d.b_f16 && !d.a_f16 && !d.packed_b && d.m <= 64 && d.n >= 8 && d.k >= 160 && d.batch <= 65535;
+}
+
+// K splits: enough workgroups for two per CU, with at least two 64-deep
+// stages each.
+W3Plan w3_plan(uint32_t cus, const ResolvedMatmul &d) {
+  W3Plan p{};
+  p.rows = d.m <= 32 ? 32 : 64;
+  p.tiles_m = div_ceil(d.m, p.rows);
+  p.tiles_n = div_ceil(d.n, TA_W3_BN);
+  p.blocks = p.tiles_m * (p.rows / 32);
+  p.ksteps = div_ceil(d.k, TA_W3_BK) * (TA_W3_BK / 16);
+  p.chunks = div_ceil(p.ksteps, TA_X6_CHUNK_STEPS);
+  p.planes = d.batch_stride_a ? d.batch : 1;
+  const uint64_t tiles = (uint64_t)d.batch * p.tiles_m * p.tiles_n;
+  const uint32_t steps = p.ksteps / (TA_W3_BK / 16);
+  const uint64_t wanted = (2ull * cus + tiles - 1) / tiles;
+  p.splits = (uint32_t)std::clamp<uint64_t>(wanted, 1, std::max(1u, steps / 2));
+  p.bits_off = p.planes * p.blocks * p.ksteps * TA_X6_STEP_BYTES;
+  p.pack_bytes = (p.bits_off + p.planes * p.chunks * p.blocks * 32 * 4 + 255) / 256 * 256;
+  p.partial_bytes = p.splits > 1 ? tiles * p.splits * p.rows * TA_W3_BN * 4 : 0;
+  p.counters = p.splits > 1 ? tiles * TA_GEMV_COUNTER_STRIDE : 0;
+  return p;
+}
+
 // splitk2.rs:226-246.
 void validate_scratch_geometry(uint32_t batch, uint32_t m, uint32_t n, uint32_t k,
                                uint32_t splits) {

@@ -1,0 +1,90 @@
+"""Few rows of f32 A on f16 weights (A in three bf16 pieces, each weight in
+two): tile and stage edges, weight rows that are and are not whole 16-byte
+pieces, K splits, batches, epilogues, a packed A shared by several ops of a
+submission, and the values that fall back on whole f32 products."""
+
+import numpy as np
+import pytest
+
+from test_gemm_gpu import check_f32
+
+pytestmark = pytest.mark.gpu
+
+
+def weights(oracle, n, seed):
+    return oracle.round_via_f16(oracle.fill_det(n, seed))
+
+
+@pytest.mark.parametrize("bt,ba,m,n,k", [(1, 1, 9, 8, 160), (1, 1, 31, 63, 161), (1, 1, 32, 64, 192), (1, 1, 33, 65, 1000),
+                                         (1, 1, 63, 374, 3060), (1, 1, 64, 40, 4096), (1, 1, 16, 4096, 256),
+                                         (3, 3, 1, 72, 300), (3, 1, 8, 130, 513), (2, 2, 40, 40, 640)])
+def test_f16w3_shapes(ta, ex, oracle, bt, ba, m, n, k):
+    sa = [m, k] if bt == 1 else [ba, m, k]
+    ha, hb = oracle.fill_det(ba * m * k, 31), weights(oracle, bt * k * n, 32)
+    hbias, hd = oracle.fill_det(n, 33), oracle.fill_det(bt * m * n, 34)
+    a = ex.tensor_from(ha, shape=sa)
+    b = ex.tensor_from(hb, shape=[k, n] if bt == 1 else [bt, k, n], f16=True)
+    bias = ex.tensor_from(hbias, shape=[n])
+    shape = [m, n] if bt == 1 else [bt, m, n]
+    d, c = ex.tensor_from(hd, shape=shape), ex.tensor(shape)
+    for epi, ref in [(ta.Epilogue(), {}),
+                     (ta.Epilogue(bias=bias, activation=ta.ACTIVATION_SILU, binary=ta.BINARY_MUL, d=d),
+                      dict(bias=hbias, act=2, binary=2, d=hd)),
+                     (ta.Epilogue(activation=ta.ACTIVATION_GELU, binary=ta.BINARY_ADD_SCALED, d=d, beta=0.5),
+                      dict(act=3, binary=1, d=hd, beta=0.5))]:
+        for _ in range(2):  # the split counters are back at zero
+            ex.upload(c, np.zeros(bt * m * n, np.float32))
+            ex.run_ops([ta.MatmulOp(a, b, c, epilogue=epi)])
+            check_f32(ex.download(c), oracle.reference_gemm(ha, hb, bt, m, n, k, **ref), k, oracle)
+
+
+def test_f16w3_accumulates(ta, ex, oracle):
+    m, n, k = 20, 96, 500
+    ha, hb, hc = oracle.fill_det(m * k, 41), weights(oracle, k * n, 42), oracle.fill_det(m * n, 43)
+    c = ex.tensor_from(hc, shape=[m, n])
+    ex.run_ops([ta.MatmulOp(ex.tensor_from(ha, shape=[m, k]), ex.tensor_from(hb, shape=[k, n], f16=True), c, alpha=0.75,
+                            accumulate=True)])
+    check_f32(ex.download(c), oracle.reference_gemm(ha, hb, 1, m, n, k, 0.75, hc, True), k, oracle)
+
+
+def test_f16w3_packed_a_is_reused_only_while_valid(ta, ex, oracle):
+    """x feeds two ops, is overwritten by the third and read again, and the
+    same memory is read at another K; graph, prepared and one-by-one agree."""
+    m, k = 24, 256
+    hx, hw = oracle.fill_det(m * k, 51), [weights(oracle, k * k, 52 + i) for i in range(3)]
+    w = [ex.tensor_from(v, shape=[k, k], f16=True) for v in hw]
+    x, y, z, u = (ex.tensor([m, k]) for _ in range(4))
+    ops = [ta.MatmulOp(x, w[0], y), ta.MatmulOp(x, w[1], z), ta.MatmulOp(y, w[2], x), ta.MatmulOp(x, w[0], u)]
+    got = []
+    prep = ex.prepare_op_graph(ops)
+    for run in (lambda: [ex.run_ops([op]) for op in ops], lambda: ex.run_op_graph(ops), prep.run, prep.run):
+        ex.upload(x, hx)
+        run()
+        got.append([ex.download(t) for t in (y, z, x, u)])
+    for other in got[1:]:
+        for p, q in zip(got[0], other):
+            assert np.array_equal(p, q)
+    y_ref = oracle.reference_gemm(hx, hw[0], 1, m, k, k)
+    check_f32(got[0][0], y_ref, k, oracle)
+    check_f32(got[0][1], oracle.reference_gemm(hx, hw[1], 1, m, k, k), k, oracle)
+    check_f32(got[0][3], oracle.reference_gemm(got[0][2].reshape(-1), hw[0], 1, m, k, k), k, oracle)
+
+
+@pytest.mark.parametrize("n", [136, 133])
+def test_f16w3_special_values(ta, ex, n):
+    """Infinities on either side, NaN and a row of tiny values give what
+    whole f32 products give."""
+    rng = np.random.default_rng(8)
+    m, k = 40, 400
+    a = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
+    b = rng.uniform(0.5, 1.5, (k, n)).astype(np.float16).astype(np.float32)
+    a[3, 5], a[7, 1], b[11, 20] = np.inf, np.nan, np.inf
+    a[12] *= np.float32(2.0 ** -115)
+    c = ex.tensor([m, n])
+    ex.run_ops([ta.MatmulOp(ex.tensor_from(a), ex.tensor_from(b, f16=True), c)])
+    got, exact = ex.download(c), a.astype(np.float64) @ b.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(exact))
+    inf = np.isinf(exact)
+    assert np.array_equal(got[inf], exact[inf].astype(np.float32))
+    fine = np.isfinite(exact)
+    assert np.max(np.abs(got[fine] - exact[fine]) / exact[fine]) <= k * 2.0 ** -24
