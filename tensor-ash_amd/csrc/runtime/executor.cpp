@@ -336,7 +336,7 @@ struct ExecutorImpl {
   // kernel selection, or a tuned kernel or split count that differs from
   // the heuristic's, runs as named.
   void choose_x6(const ResolvedMatmul &d, OpPlan &plan) const {
-    if (!selection.is_auto() || d.a_f16 || d.b_f16 || d.packed_b)
+    if (!selection.is_auto() || KERNEL_SPECS[plan.kernel].kind != KernelKind::GemmF32)
       return;
     const uint32_t cus = ctx->cu_count();
     const size_t heur = heuristic_kernel_index(cus, d.batch, d.m, d.n, d.k, false, false);

@@ -134,3 +134,28 @@ def test_cpp_mirror_unit_tests(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "all passed" in r.stdout
+
+
+def test_ops_array_packs_what_the_structures_hold(ta):
+    """The packed operation arrays equal the ctypes structures built field
+    by field, for every version and for values that do not pack."""
+    import ctypes
+
+    class T:
+        def __init__(self, h):
+            self.handle = h
+
+    t = [T(0x7F0000001000 + 64 * i) for i in range(5)]
+    full = ta.MatmulOp(t[0], t[1], t[2], 0.5, True, ta.Epilogue(t[3], 2, 1, t[4], 0.25))
+    plain = ta.MatmulOp(t[0], t[1], t[2])
+    packed = ta.MatmulOp(t[0], t[1], t[2], packed_b=True)
+    normed = ta.MatmulOp(t[0], t[1], t[2], normed_a=(t[3], 1e-5))
+    closed = ta.MatmulOp(T(None), t[1], t[2])
+    odd = ta.MatmulOp(t[0], t[1], t[2], np.float32(0.5), np.bool_(True))
+    for ops, version in [([full, plain], 1), ([plain, packed, full], 2), ([full, normed], 3), ([closed, plain], 1),
+                         ([closed, normed], 3), ([odd], 1), ([odd, packed], 2), ([plain], 1)]:
+        arr, got = ta._ops_array(ops)
+        assert got == version and len(arr) == len(ops)
+        for a, op in zip(arr, ops):
+            want = {1: op._raw, 2: lambda: ta._OpV2(op._raw(), int(op.packed_b)), 3: op._raw_v3}[version]()
+            assert ctypes.string_at(ctypes.byref(a), ctypes.sizeof(a)) == bytes(want)
