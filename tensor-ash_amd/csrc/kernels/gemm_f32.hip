@@ -308,6 +308,92 @@ template <int BM, int BN, int WGM, int WGN, int NS> struct GemmF32Mi16 {
   }
 };
 
+// One output tile by G groups of waves, each over a G-th of K (in whole
+// slabs), for launches whose tiles leave CUs or wave slots empty: a tile's
+// time is its chain of slabs (load, LDS, 32 MFMAs), and G chains side by
+// side are G times shorter.  The groups' sums meet in LDS, in group order.
+// Bound by the slabs' latencies: 512^3 (64 tiles) 16.2 us against 20.7 with
+// one group, 512 x 2048 x 2048 48.6 against 66.5.
+template <int BM, int BN, int WGM, int WGN, bool VEC, int G> struct GemmF32Groups {
+  typedef GemmF32<BM, BN, WGM, WGN, VEC, false, 16> Tile;
+  static constexpr int T = Tile::T, FM = Tile::FM, FN = Tile::FN, BK = Tile::BK, WT = WGM * WGN;
+  static constexpr int SMEM_FLOATS = G * Tile::SMEM_FLOATS;
+  static_assert((G - 1) * WT * FM * FN * 1024 <= SMEM_FLOATS, "the groups' sums fit in LDS");
+
+  static TA_DEVICE void run(const GemmArgs &p) {
+    __shared__ __attribute__((aligned(16))) float smem[SMEM_FLOATS];
+    const uint32_t tid = threadIdx.x % T, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t group = __builtin_amdgcn_readfirstlane(threadIdx.x / T);
+    const uint32_t wm = wave / WGN, wn = wave % WGN;
+    uint32_t tm, tn;
+    ta_tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    const uint32_t m0 = tm * BM, n0 = tn * BN, batch = blockIdx.z;
+    const float *A = static_cast<const float *>(p.a) + (uint64_t)batch * p.stride_a;
+    const float *B = static_cast<const float *>(p.b) + (uint64_t)batch * p.stride_b;
+    const bool mn_full = (m0 + BM <= p.m) && (n0 + BN <= p.n);
+    // Every group walks `per` slabs; those past its window are zeros.
+    const uint32_t per = ((p.k + BK - 1) / BK + G - 1) / G;
+    const uint32_t klo = min(group * per * BK, p.k), khi = min(klo + per * BK, p.k);
+    float *own = smem + group * Tile::SMEM_FLOATS;
+
+    f32x16 acc[FM][FN];
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+        acc[fm][fn] = f32x16{};
+    // AHEAD slabs are on their way in registers: with few slabs per group the
+    // memory latency, not the work, is what a slab would wait for.
+    constexpr int AHEAD = 4;
+    f32x4 ra[AHEAD][Tile::A_PER], rb[AHEAD][Tile::B_PER];
+    auto load = [&](uint32_t i, f32x4 (&a)[Tile::A_PER], f32x4 (&b)[Tile::B_PER]) __attribute__((always_inline)) {
+      const uint32_t k0 = klo + i * BK;
+      const bool full = mn_full && k0 + BK <= khi;
+      Tile::load_a(A, p.m, p.k, m0, k0, klo, khi, full, tid, a);
+      Tile::load_b(B, p.n, n0, k0, klo, khi, full, tid, b);
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      load(j, ra[j], rb[j]);
+    for (uint32_t i0 = 0; i0 < per; i0 += AHEAD) {
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        const uint32_t i = i0 + j;
+        if (i >= per)
+          break;
+        // The other buffer's readers passed the barrier of slab i - 1's write.
+        float *cur = own + (j & 1) * (Tile::A_STAGE + Tile::B_STAGE);
+        Tile::store_lds(cur, cur + Tile::A_STAGE, tid, ra[j], rb[j]);
+        __syncthreads();
+        if (i + AHEAD < per)
+          load(i + AHEAD, ra[j], rb[j]);
+        Tile::compute(cur, cur + Tile::A_STAGE, lane, wm, wn, acc);
+      }
+    }
+    __syncthreads();
+    if (group > 0) {
+#pragma unroll
+      for (int f = 0; f < FM * FN; ++f)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          smem[(((group - 1) * WT + wave) * FM * FN + f) * 1024 + r * 64 + lane] = acc[f / FN][f % FN][r];
+    }
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int g = 1; g < G; ++g)
+#pragma unroll
+        for (int f = 0; f < FM * FN; ++f)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[f / FN][f % FN][r] += smem[(((g - 1) * WT + wave) * FM * FN + f) * 1024 + r * 64 + lane];
+    }
+    __syncthreads();
+    ta_store_tile<Tile::WTM, Tile::WTN, FM, FN, T, false>(smem, SMEM_FLOATS, acc, p, lane, wave, wm, wn, m0,
+                                                          n0, batch, 0, group == 0);
+  }
+};
+
 } // namespace
 
 #define TA_GEMM_F32(NAME, BM, BN, WGM, WGN, VEC, HALF_B, BK)                      \
@@ -333,6 +419,13 @@ TA_GEMM_F32_FAMILY(m64n64, 64, 64, 2, 2, 16)
 TA_GEMM_F32_FAMILY(m64n256, 64, 256, 1, 4, 16)
 TA_GEMM_F32_FAMILY(m32n128, 32, 128, 1, 2, 16)
 TA_GEMM_F32_FAMILY(m32n64, 32, 64, 1, 2, 16)
+
+extern "C" __global__ __launch_bounds__(1024) void ta_gemm_f32_m64n64_k4_vec(GemmArgs p) {
+  GemmF32Groups<64, 64, 2, 2, true, 4>::run(p);
+}
+extern "C" __global__ __launch_bounds__(1024) void ta_gemm_f32_m64n64_k4_gen(GemmArgs p) {
+  GemmF32Groups<64, 64, 2, 2, false, 4>::run(p);
+}
 
 // Whole tiles of f32 A and B whose K windows hold multiples of 64 rows
 // (see GemmF32Mi16): the 256x256 data-parallel tile and the split-K

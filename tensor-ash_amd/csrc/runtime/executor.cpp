@@ -805,10 +805,16 @@ struct ExecutorImpl {
     const bool vec = d.k % 4 == 0 && d.n % 4 == 0;
     const bool mi16 = s.kind == KernelKind::GemmF32 && f32_mi16_ok(d, s.tile_m, s.tile_n,
                                                                    a.num_splits);
-    const uint32_t threads = mi16  ? mi16_threads(s.tile_m)
-                             : lds ? lds_threads
-                                   : gemm_threads(s);
-    launch(std::string(s.symbol) + (mi16 ? "_mi16" : lds ? "_lds" : vec ? "_vec" : "_gen"),
+    const bool groups = !mi16 && f32_groups_ok(ctx->cu_count(), d, s, a.num_splits);
+    const uint32_t threads = mi16     ? mi16_threads(s.tile_m)
+                             : lds    ? lds_threads
+                             : groups ? 1024u
+                                      : gemm_threads(s);
+    launch(std::string(s.symbol) + (groups ? "_k4" : "") +
+               (mi16  ? "_mi16"
+                : lds ? "_lds"
+                : vec ? "_vec"
+                      : "_gen"),
            (uint32_t)gx, 1, (uint32_t)gz, threads, &a, stream);
     if (splits > 1) {
       SplitReduceArgs r{};

@@ -140,6 +140,16 @@ bool f32_mi16_ok(const ResolvedMatmul &d, uint32_t tile_m, uint32_t tile_n, uint
          16ull * d.n * 4 < (1ull << 32);
 }
 
+// The four-K-group form of the 64 x 64 FP32 tile (ta_gemm_f32_m64n64_k4_*):
+// while the tiles fit the CUs once, a tile's chain of K slabs is the time.
+// us, four groups / one: 512^3 16.2 / 20.7, 512x2048x2048 48.6 / 66.5,
+// 300x520x500 25.0 / 36.2, 160x1488x268 16.9 / 21.4; K = 128: 9.4 / 9.0.
+bool f32_groups_ok(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &s, uint32_t planes) {
+  return s.kind == KernelKind::GemmF32 && s.tile_m == 64 && s.tile_n == 64 && planes == 1 && !d.b_f16 &&
+         !d.a_f16 && d.k >= 160 && !std::getenv("TA_NO_F32_GROUPS") &&
+         (uint64_t)d.batch * div_ceil(d.m, 64) * div_ceil(d.n, 64) <= cus;
+}
+
 bool kernel_supports(const KernelSpec &s, const ResolvedMatmul &d) {
   // The 256x256 f16-MFMA tiles exist only as pipelined kernels.
   if ((s.kind == KernelKind::GemmF16Mfma || s.kind == KernelKind::GemmA16) && s.tile_m == 256 &&
@@ -421,8 +431,8 @@ F32X6Plan f32x6_plan(const ResolvedMatmul &d, uint32_t tile) {
 // 0.21 (64 x 64, four): 4096^3 561 us on 256 tiles, 3000^3 331 us and
 // 2048^3 93 us on 128 x 128, 512x2048x2048 30 us on 64 x 64.
 // FP32 MFMA: 3.6 us per k-step and round for whole 256 x 256 tiles, 2.0 /
-// 1.4 / 0.8 / 0.52 for the smaller ones; tiles that cross the matrix's edge
-// load scalars, and the launch waits for them (3000^3 on 256 x 128: 6.4 us;
+// 1.4 / 0.8 / 0.52 for the smaller ones (64 x 64 in four K groups 0.36, at
+// an edge 0.7); tiles that cross the matrix's edge load scalars, and the launch waits for them (3000^3 on 256 x 128: 6.4 us;
 // 1000x1531x777 on 64 x 64: 1.0).  Split-K: 75 TFLOP/s plus 10 us.
 uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &fp32,
                     std::optional<uint32_t> splits) {
@@ -440,6 +450,7 @@ uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &fp3
                         : area >= 256 * 128 ? (whole ? 2.0 : 6.4)
                         : area >= 128 * 128 ? (whole ? 1.4 : 3.2)
                         : area >= 128 * 64  ? (whole ? 0.8 : 1.8)
+                        : f32_groups_ok(cus, d, fp32, 1) ? (whole ? 0.36 : 0.7)
                                             : (whole ? 0.52 : 1.0);
     const double tiles = (double)d.batch * div_ceil(d.m, fp32.tile_m) * div_ceil(d.n, fp32.tile_n);
     const double rounds = area >= 128 * 128 ? std::ceil(tiles / cus) : std::max(1.0, tiles / cus);
