@@ -428,41 +428,51 @@ F32X6Plan f32x6_plan(const ResolvedMatmul &d, uint32_t tile) {
 // Split products: the pack (one launch: 6.5 us, 10 B per element at 5.5
 // TB/s), the gap to the GEMM and its ramp, then rounds of tiles, each k-step
 // (16) of a round at 2.2 us (256 x 256), 0.6 (128 x 128, two K groups) or
-// 0.21 (64 x 64, four): 4096^3 561 us on 256 tiles, 3000^3 331 us and
+// 0.13 to 0.21 as the CUs fill (64 x 64, four; 25 tiles 0.14, 144 0.17, 256
+// 0.21): 4096^3 561 us on 256 tiles, 3000^3 331 us and
 // 2048^3 93 us on 128 x 128, 512x2048x2048 30 us on 64 x 64.
 // FP32 MFMA: 3.6 us per k-step and round for whole 256 x 256 tiles, 2.0 /
 // 1.4 / 0.8 / 0.52 for the smaller ones (64 x 64 in four K groups 0.36, at
-// an edge 0.7); tiles that cross the matrix's edge load scalars, and the launch waits for them (3000^3 on 256 x 128: 6.4 us;
-// 1000x1531x777 on 64 x 64: 1.0).  Split-K: 75 TFLOP/s plus 10 us.
+// an edge 0.7); tiles that cross the matrix's edge load scalars, and the
+// launch waits for them (3000^3 on 256 x 128: 6.4 us; 1000x1531x777 on
+// 64 x 64: 1.0).  Split-K adds 10 us for its second stage; its steps cost the
+// same (1536x360x1336 in 4 windows 73.6 us, 64 x 64 split products 30.2;
+// 500x400x3000 in 8 82.4 / 43.8), except whole tiles and windows, which run at
+// 75 TFLOP/s (512x512x4096 27.5 / 53.7).
 uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &fp32,
                     std::optional<uint32_t> splits) {
   if (d.a_f16 || d.b_f16 || d.packed_b || fp32.kind != KernelKind::GemmF32 || d.batch > 65535 ||
       d.m < 32 || d.n < 32 || d.k < 64)
     return 0;
   const double ksteps = (d.k + 15) / 16;
+  const bool whole = d.m % fp32.tile_m == 0 && d.n % fp32.tile_n == 0;
+  const uint32_t planes = splits ? *splits * splitk_sub_splits(cus, d, *splits) : 1;
   double old_us;
-  if (splits) {
+  if (splits && whole && f32_mi16_ok(d, fp32.tile_m, fp32.tile_n, planes)) {
     old_us = 10.0 + (double)d.total_flops / 75e6;
   } else {
-    const bool whole = d.m % fp32.tile_m == 0 && d.n % fp32.tile_n == 0;
     const uint32_t area = fp32.tile_m * fp32.tile_n;
     const double step = area >= 256 * 256   ? (whole ? 3.6 : 9.0)
                         : area >= 256 * 128 ? (whole ? 2.0 : 6.4)
                         : area >= 128 * 128 ? (whole ? 1.4 : 3.2)
                         : area >= 128 * 64  ? (whole ? 0.8 : 1.8)
-                        : f32_groups_ok(cus, d, fp32, 1) ? (whole ? 0.36 : 0.7)
+                        : f32_groups_ok(cus, d, fp32, planes) ? (whole ? 0.36 : 0.7)
                                             : (whole ? 0.52 : 1.0);
-    const double tiles = (double)d.batch * div_ceil(d.m, fp32.tile_m) * div_ceil(d.n, fp32.tile_n);
+    const double tiles =
+        (double)planes * d.batch * div_ceil(d.m, fp32.tile_m) * div_ceil(d.n, fp32.tile_n);
     const double rounds = area >= 128 * 128 ? std::ceil(tiles / cus) : std::max(1.0, tiles / cus);
-    old_us = 3.0 + rounds * ksteps * step;
+    old_us = (splits ? 10.0 : 3.0) + rounds * ksteps / planes * step;
   }
   const double planes_a = d.batch_stride_a ? d.batch : 1, planes_b = d.batch_stride_b ? d.batch : 1;
   const double pack_us =
       6.5 + 10.0 * d.k * (planes_a * (double)d.m + planes_b * (double)d.n) / 5.5e6;
   uint32_t best = 0;
   double best_us = 0.95 * old_us;
-  for (const auto &[tile, step] : {std::pair<uint32_t, double>{256, 2.2}, {128, 0.6}, {64, 0.21}}) {
+  for (const uint32_t tile : {256u, 128u, 64u}) {
     const double tiles = (double)d.batch * div_ceil(d.m, tile) * div_ceil(d.n, tile);
+    const double step = tile == 256   ? 2.2
+                        : tile == 128 ? 0.6
+                                      : 0.13 + 0.08 * std::min(1.0, tiles / cus);
     const double us = pack_us + 5.0 + std::ceil(tiles / cus) * ksteps * step;
     if (us < best_us && f32x6_plan(d, tile).bytes <= kF32X6ScratchCapBytes) {
       best_us = us;

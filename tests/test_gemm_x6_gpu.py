@@ -106,3 +106,17 @@ def test_x6_in_graphs_and_prepared(ta, ex, oracle, monkeypatch):
         ex.upload(z, np.zeros((m, k), np.float32))
         run()
         assert np.array_equal(ex.download(z), alone)
+
+
+@pytest.mark.parametrize("m,n,k,form", [(500, 400, 3000, 64), (640, 320, 1600, 64), (512, 512, 4096, 0)])
+def test_deep_k_route(ta, ex, oracle, monkeypatch, m, n, k, form):
+    """Ragged tiles or K windows leave split-K for the split products; whole
+    ones stay.  Same bits as the form named, and right against the oracle."""
+    run_case(ta, ex, oracle, m, n, k)
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    named = product(ta, ex, a, b, monkeypatch, form)
+    monkeypatch.delenv("TA_F32X6")
+    ta_, tb, c = ex.tensor_from(a), ex.tensor_from(b), ex.tensor([m, n])
+    ex.run_ops([ta.MatmulOp(ta_, tb, c)])
+    assert np.array_equal(ex.download(c), named)
