@@ -387,7 +387,7 @@ def _ops_array(ops: Sequence[MatmulOp]):
             e, packed = o.epilogue, bool(o.packed_b)
             v2 = v2 or packed
             bias, d = e.bias, e.d
-            pack(buf, i * size, o.a.handle, o.b.handle, o.c.handle, o.alpha, o.accumulate,
+            pack(buf, i * size, o.a.handle, o.b.handle, o.c.handle, o.alpha, int(o.accumulate),
                  bias.handle if bias is not None and bias else 0, e.activation, e.binary,
                  d.handle if d is not None and d else 0, e.beta, packed)
     except struct.error:  # no handle (a closed tensor: the C call reports the null), or no plain number
