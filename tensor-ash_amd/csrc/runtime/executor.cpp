@@ -452,65 +452,6 @@ struct ExecutorImpl {
     return (planes * d.m * d.k * 2 + 255) / 256 * 256;
   }
 
-  // f16 copies of A that pre-passes (or a dual launch's f16 output copy)
-  // of a submission left behind: a later f16w GEMM with the same A (same
-  // buffer, same elements) reuses one unless an op in between wrote that
-  // buffer, or wrote the split-K region the copy lives in (record() and
-  // launch_gemm() drop such entries).  Two entries, so a layer that
-  // converts x for QKV and then the attention output for O still finds x
-  // for its up/gate pair.  Pre-pass copies go to the half of the split-K
-  // region the other live copy does not use (scratch_need reserves two
-  // halves, each as large as the op's A).
-  struct CvtEntry {
-    const void *buffer = nullptr;
-    const void *src = nullptr;
-    uint64_t n = 0;
-    void *base = nullptr;       // where the copy lives
-    size_t producer = SIZE_MAX; // op whose epilogue wrote it, if any
-    int half = -1;              // split-K region half, -1 = elsewhere
-    uint32_t packed_k = 0;      // f16 copy: 0; packed pieces (ta_pack_f32x3): their K
-    uint64_t age = 0;
-  };
-  struct CvtCache {
-    CvtEntry e[2];
-    uint64_t clock = 0;
-    CvtEntry *find(const void *buffer, const void *src, uint64_t n, uint32_t packed_k = 0) {
-      for (auto &x : e)
-        if (x.buffer && x.buffer == buffer && x.src == src && x.n == n && x.packed_k == packed_k)
-          return &x;
-      return nullptr;
-    }
-    // The entry to replace: an empty one, else the older.
-    CvtEntry &victim() {
-      if (!e[0].buffer)
-        return e[0];
-      if (!e[1].buffer)
-        return e[1];
-      return e[0].age <= e[1].age ? e[0] : e[1];
-    }
-    // A copy written at `v.base` replaces whatever entry that memory held
-    // (every dual launch writes its f16 output copy to the same scratch).
-    void put(CvtEntry &slot, CvtEntry v) {
-      for (auto &x : e)
-        if (&x != &slot && x.buffer && x.base == v.base)
-          x = CvtEntry{};
-      v.age = ++clock;
-      slot = v;
-    }
-    // An op wrote `buffer`: copies of it are stale (except the one that
-    // op's own epilogue produced).
-    void wrote(const void *buffer, size_t op) {
-      for (auto &x : e)
-        if (x.buffer && x.buffer == buffer && x.producer != op)
-          x = CvtEntry{};
-    }
-    void drop_region() { // the split-K region was overwritten
-      for (auto &x : e)
-        if (x.half >= 0)
-          x = CvtEntry{};
-    }
-  };
-
   // Does op i take the f32 -> f16 pre-pass of its A (the pipelined f16w
   // route; not a16, whose A is f16 already)?
   bool converts_a(const ResolvedMatmul &d, const OpPlan &p) const {
@@ -623,10 +564,9 @@ struct ExecutorImpl {
     if (scratch.partial_bytes < w.partial_bytes || scratch.counters_len < w.counters)
       fail("internal: split-product scratch not reserved");
     const void *buf = op.call.a->buffer_id();
-    // rows x K of one plane, its planes and its padding decide the layout
     const uint64_t n = w.planes * d.m * d.k;
     char *packed = nullptr;
-    if (CvtEntry *hit = cvt.find(buf, a.a, n, d.k)) {
+    if (CvtEntry *hit = cvt.find(buf, a.a, n, w.planes, d.m)) {
       packed = static_cast<char *>(hit->base);
     } else {
       CvtEntry &v = cvt.victim();
@@ -641,7 +581,8 @@ struct ExecutorImpl {
                       w.chunks, 1, w.planes);
       launch("ta_pack_f32x3", pk.a.groups, 1, 1, 256, &pk, stream);
       CvtEntry e{buf, a.a, n, packed, SIZE_MAX, half};
-      e.packed_k = d.k;
+      e.planes = w.planes;
+      e.rows = d.m;
       cvt.put(v, e);
     }
     GemmW3Args g{};

@@ -128,6 +128,73 @@ uint32_t gemv_unit(uint32_t tw, bool f32_weights, bool dual, uint32_t rows);
 GemvPlan plan_gemv(uint32_t cus, uint32_t rows, uint32_t n, uint32_t k, uint32_t tw, bool dual,
                    uint32_t unit);
 
+// ---- copies of A kept within a submission ----
+// f16 copies of A that pre-passes (or a dual launch's f16 output copy) of a
+// submission left behind: a later f16w GEMM with the same A (same buffer,
+// same elements) reuses one unless an op in between wrote that buffer, or
+// wrote the split-K region the copy lives in (record() and launch_gemm()
+// drop such entries).  Two entries, so a layer that converts x for QKV and
+// then the attention output for O still finds x for its up/gate pair.
+// Pre-pass copies go to the half of the split-K region the other live copy
+// does not use (scratch_need reserves two halves, each as large as the op's
+// A).
+// A's packed pieces (ta_pack_f32x3) are kept the same way.  An f16 copy has
+// A's own order, whatever shape an alias gives the buffer; the pieces lie
+// in blocks of 32 rows that start anew in every plane, so they are the same
+// only for the same planes of the same rows (n then fixes K).
+struct CvtEntry {
+  const void *buffer = nullptr;
+  const void *src = nullptr;
+  uint64_t n = 0;             // elements of A
+  void *base = nullptr;       // where the copy lives
+  size_t producer = SIZE_MAX; // op whose epilogue wrote it, if any
+  int half = -1;              // split-K region half, -1 = elsewhere
+  uint64_t planes = 0;        // packed pieces: planes and rows of each;
+  uint32_t rows = 0;          // f16 copy: 0
+  uint64_t age = 0;
+};
+struct CvtCache {
+  CvtEntry e[2];
+  uint64_t clock = 0;
+  CvtEntry *find(const void *buffer, const void *src, uint64_t n, uint64_t planes = 0,
+                 uint32_t rows = 0) {
+    for (auto &x : e)
+      if (x.buffer && x.buffer == buffer && x.src == src && x.n == n && x.planes == planes &&
+          x.rows == rows)
+        return &x;
+    return nullptr;
+  }
+  // The entry to replace: an empty one, else the older.
+  CvtEntry &victim() {
+    if (!e[0].buffer)
+      return e[0];
+    if (!e[1].buffer)
+      return e[1];
+    return e[0].age <= e[1].age ? e[0] : e[1];
+  }
+  // A copy written at `v.base` replaces whatever entry that memory held
+  // (every dual launch writes its f16 output copy to the same scratch).
+  void put(CvtEntry &slot, CvtEntry v) {
+    for (auto &x : e)
+      if (&x != &slot && x.buffer && x.base == v.base)
+        x = CvtEntry{};
+    v.age = ++clock;
+    slot = v;
+  }
+  // An op wrote `buffer`: copies of it are stale (except the one that
+  // op's own epilogue produced).
+  void wrote(const void *buffer, size_t op) {
+    for (auto &x : e)
+      if (x.buffer && x.buffer == buffer && x.producer != op)
+        x = CvtEntry{};
+  }
+  void drop_region() { // the split-K region was overwritten
+    for (auto &x : e)
+      if (x.half >= 0)
+        x = CvtEntry{};
+  }
+};
+
 // ---- f16w A conversions converted up front ----
 // One op of a submission as the paired up-front conversion sees it: its A
 // (buffer, device pointer, values converted), whether its route converts A

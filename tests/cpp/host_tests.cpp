@@ -352,6 +352,37 @@ static void test_paired_conversion_picks() {
   CHECK(paired_conversion_picks({}).empty());
 }
 
+// Packed pieces of A are found again only under the planes and rows they
+// were packed for: aliases of one buffer have the same element count.
+static void test_packed_a_key() {
+  int buf = 0, out = 0;
+  const uint64_t n = 32 * 512;
+  CvtCache c;
+  CvtEntry e{&buf, &buf, n, &out, SIZE_MAX, 0};
+  e.planes = 1, e.rows = 32;
+  c.put(c.victim(), e);
+  CHECK(c.find(&buf, &buf, n, 1, 32) && c.find(&buf, &buf, n, 1, 32)->base == &out);
+  CHECK(!c.find(&buf, &buf, n, 2, 16)); // [2, 16, K] over [32, K]
+  CHECK(!c.find(&buf, &buf, n, 1, 16)); // [16, 2 K]
+  CHECK(!c.find(&buf, &buf, n, 32, 1));
+  CHECK(!c.find(&buf, &buf, n)); // no f16 copy
+  CvtEntry f{&buf, &buf, n, &buf, SIZE_MAX, 1};
+  c.put(c.victim(), f);
+  CHECK(c.find(&buf, &buf, n) && c.find(&buf, &buf, n)->base == &buf);
+  CHECK(c.find(&buf, &buf, n, 1, 32)->base == &out);
+  // both views below take the route that keeps packed pieces
+  for (const auto &d : {ResolvedMatmul::from_shapes({32, 512}, {512, 96}, {32, 96}),
+                        ResolvedMatmul::from_shapes({2, 16, 512}, {2, 512, 96}, {2, 16, 96})}) {
+    ResolvedMatmul h = d;
+    h.b_f16 = true;
+    CHECK(KERNEL_SPECS[heuristic_kernel_index(256, h.batch, h.m, h.n, h.k, true, false)].kind ==
+          KernelKind::GemmF16w);
+    CHECK(w3_ok(h));
+  }
+  c.wrote(&buf, 3);
+  CHECK(!c.find(&buf, &buf, n) && !c.find(&buf, &buf, n, 1, 32));
+}
+
 int main() {
   test_resolution();
   test_registry();
@@ -361,6 +392,7 @@ int main() {
   test_tuner_helpers();
   test_dtype();
   test_paired_conversion_picks();
+  test_packed_a_key();
   std::printf("%d checks, %d failed\n", g_pass + g_fail, g_fail);
   if (g_fail == 0)
     std::printf("all passed\n");

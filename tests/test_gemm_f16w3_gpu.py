@@ -3,6 +3,9 @@ two): tile and stage edges, weight rows that are and are not whole 16-byte
 pieces, K splits, batches, epilogues, a packed A shared by several ops of a
 submission, and the values that fall back on whole f32 products."""
 
+import subprocess
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -48,8 +51,8 @@ def test_f16w3_accumulates(ta, ex, oracle):
 
 
 def test_f16w3_packed_a_is_reused_only_while_valid(ta, ex, oracle):
-    """x feeds two ops, is overwritten by the third and read again, and the
-    same memory is read at another K; graph, prepared and one-by-one agree."""
+    """x feeds two ops, is overwritten by the third and read again; graph,
+    prepared and one-by-one agree."""
     m, k = 24, 256
     hx, hw = oracle.fill_det(m * k, 51), [weights(oracle, k * k, 52 + i) for i in range(3)]
     w = [ex.tensor_from(v, shape=[k, k], f16=True) for v in hw]
@@ -68,6 +71,19 @@ def test_f16w3_packed_a_is_reused_only_while_valid(ta, ex, oracle):
     check_f32(got[0][0], y_ref, k, oracle)
     check_f32(got[0][1], oracle.reference_gemm(hx, hw[1], 1, m, k, k), k, oracle)
     check_f32(got[0][3], oracle.reference_gemm(got[0][2].reshape(-1), hw[0], 1, m, k, k), k, oracle)
+
+
+def test_f16w3_packed_a_under_other_shapes(tmp_path):
+    """One buffer read as [32, K], [2, 16, K], [16, 2 K] and [4, 16, K / 2] by
+    two ops of a submission, every pair in both orders (tests/cpp/alias_tests.cpp:
+    aliases are a C++ interface), against sums in f64."""
+    root = Path(__file__).resolve().parent.parent
+    lib, exe = root / "tensor-ash_amd" / "lib", tmp_path / "alias_tests"
+    subprocess.run(["g++", "-std=c++17", "-O2", str(root / "tests" / "cpp" / "alias_tests.cpp"), "-o", str(exe),
+                    f"-L{lib}", "-ltensor_ash", f"-Wl,-rpath,{lib}", "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib"],
+                   check=True, capture_output=True, text=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
 
 
 @pytest.mark.parametrize("n", [136, 133])
