@@ -418,10 +418,17 @@ struct ExecutorImpl {
     if (p.x6) {
       need.splitk = f32x6_plan(d, p.x6).bytes;
     } else if (p.w3) {
-      const W3Plan w = w3_plan(ctx->cu_count(), d);
-      need.splitk = 2 * w.pack_bytes; // two packed A's (CvtCache)
-      need.partial = w.partial_bytes;
-      need.counters = w.counters;
+      const uint32_t group = w3_group(d);
+      for (const uint32_t planes : {group, d.batch % group}) { // whole groups, the rest
+        if (planes == 0)
+          continue;
+        const W3Plan w = w3_plan(ctx->cu_count(), w3_part(d, planes));
+        ScratchNeed part;
+        part.splitk = 2 * w.pack_bytes; // two packed A's (CvtCache)
+        part.partial = w.partial_bytes;
+        part.counters = w.counters;
+        need.merge(part);
+      }
     } else if (p.splitk2) {
       need.splitk = (uint64_t)d.batch * d.m * d.n * *p.splitk2 *
                     splitk_sub_splits(ctx->cu_count(), d, *p.splitk2) * 4;
@@ -556,10 +563,34 @@ struct ExecutorImpl {
     return j;
   }
 
+  // `planes` planes of a batch on the few-rows route.  A batch whose packed
+  // A's would pass kW3ScratchCapBytes runs in groups of planes, one after
+  // the other in the same scratch.
+  static ResolvedMatmul w3_part(ResolvedMatmul d, uint32_t planes) {
+    d.batch = planes;
+    return d;
+  }
+  void launch_w3(const ResolvedMatmul &d, const MatmulOp &op, const GemmArgs &a, Scratch &scratch,
+                 CvtCache &cvt, hipStream_t stream) const {
+    const uint32_t group = w3_group(d);
+    for (uint32_t p0 = 0; p0 < d.batch; p0 += group) {
+      GemmArgs g = a; // its stride fields are zero where an operand is broadcast
+      const uint64_t p = p0;
+      g.a = static_cast<const float *>(a.a) + p * a.stride_a;
+      g.b = static_cast<const uint16_t *>(a.b) + p * a.stride_b;
+      g.c += p * a.stride_c;
+      if (g.bias)
+        g.bias += p * a.bias_batch_stride;
+      if (g.d)
+        g.d += p * a.stride_c;
+      launch_w3_group(w3_part(d, std::min(group, d.batch - p0)), op, g, scratch, cvt, stream);
+    }
+  }
+
   // Few rows of f32 A on f16 weights: pack A (once per distinct A of a
   // submission, kept like the f16 copies), then multiply.
-  void launch_w3(const ResolvedMatmul &d, const MatmulOp &op, GemmArgs &a, Scratch &scratch,
-                 CvtCache &cvt, hipStream_t stream) const {
+  void launch_w3_group(const ResolvedMatmul &d, const MatmulOp &op, GemmArgs &a, Scratch &scratch,
+                       CvtCache &cvt, hipStream_t stream) const {
     const W3Plan w = w3_plan(ctx->cu_count(), d);
     if (scratch.partial_bytes < w.partial_bytes || scratch.counters_len < w.counters)
       fail("internal: split-product scratch not reserved");

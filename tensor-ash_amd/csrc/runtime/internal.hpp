@@ -119,6 +119,8 @@ struct W3Plan {
 };
 W3Plan w3_plan(uint32_t cus, const ResolvedMatmul &dims);
 bool w3_ok(const ResolvedMatmul &dims);
+uint32_t w3_group(const ResolvedMatmul &dims);
+constexpr uint64_t kW3ScratchCapBytes = 256ull << 20;
 
 struct GemvPlan {
   uint32_t tw = 64, mr = 1, tiles = 0, kchunk = 0, kchunks = 1;

@@ -487,9 +487,28 @@ uint32_t f32x6_tile(uint32_t cus, const ResolvedMatmul &d, const KernelSpec &fp3
 // With more rows and at least 64 columns the f16-MFMA route rounds A.  Below
 // 160 rows of K the pack's launch costs more than it saves (us, split / FP32
 // MFMA: K = 110, 33 x 5007: 16.4 / 14.6; K = 64: 10.7 / 9.0; K = 500, 40 x
-// 300: 25 / 39).
+// 300: 25 / 39).  A plane's rows are packed to blocks of 32, which stays the
+// faster form for single rows too (us, split / FP32 MFMA: 64 x 1 x 64 x 1024:
+// 22 / 68; 1024 x 1 x 64 x 1024: 94 / 1258).
 bool w3_ok(const ResolvedMatmul &d) {
-  return d.b_f16 && !d.a_f16 && !d.packed_b && d.m <= 64 && d.n >= 8 && d.k >= 160 && d.batch <= 65535;
+  return d.b_f16 && !d.a_f16 && !d.packed_b && d.m <= 64 && d.n >= 8 && d.k >= 160 && d.batch <= 65535 &&
+         w3_group(d) > 0;
+}
+
+// Planes of a batch one launch takes: two packed A's (CvtCache) stay within
+// kW3ScratchCapBytes, and the groups are of one size up to the last.  0: not
+// even one plane fits.
+uint32_t w3_group(const ResolvedMatmul &d) {
+  ResolvedMatmul one = d;
+  one.batch = 1;
+  const uint64_t plane = w3_plan(1, one).pack_bytes;
+  const uint64_t fit = kW3ScratchCapBytes / 2 / plane;
+  if (fit == 0)
+    return 0;
+  if (!d.batch_stride_a || d.batch <= fit)
+    return d.batch;
+  const uint32_t groups = (uint32_t)((d.batch + fit - 1) / fit);
+  return div_ceil(d.batch, groups);
 }
 
 // K splits: enough workgroups for two per CU, with at least two 64-deep

@@ -2,6 +2,7 @@
 // unit tests: src/matmul/tests.rs:4-165, src/pipeline/catalog.rs:384-493,
 // src/executor/splitk2.rs:472-607, src/executor/tuning.rs:319-345,
 // src/dtype.rs:114-164.  Built and run by tests/test_capi_cpu.py.
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <functional>
@@ -383,6 +384,33 @@ static void test_packed_a_key() {
   CHECK(!c.find(&buf, &buf, n) && !c.find(&buf, &buf, n, 1, 32));
 }
 
+// Scratch of the few-rows route stays under its cap for any batch: larger
+// ones run in groups of planes.
+static void test_w3_scratch() {
+  for (const auto &[b, m, n, k] : {std::array<uint32_t, 4>{1, 64, 4096, 14336}, {8, 9, 64, 160}, {400, 1, 8, 4096},
+                                   {1024, 1, 512, 4096}, {65535, 1, 8, 4096}, {30000, 1, 8, 14336}, {3, 64, 64, 300000}}) {
+    ResolvedMatmul d = ResolvedMatmul::from_shapes({b, m, k}, {b, k, n}, {b, m, n});
+    d.b_f16 = true;
+    CHECK(w3_ok(d));
+    const uint32_t group = w3_group(d);
+    CHECK(group >= 1 && group <= b);
+    ResolvedMatmul part = d;
+    part.batch = group;
+    CHECK(2 * w3_plan(256, part).pack_bytes <= kW3ScratchCapBytes);
+    // no group is much smaller than the others, and no more groups than needed
+    const uint64_t whole = 2 * w3_plan(256, d).pack_bytes, groups = (b + group - 1) / group;
+    CHECK(group * (groups - 1) < b && (groups == 1) == (whole <= kW3ScratchCapBytes));
+  }
+  // one plane that does not fit keeps the FP32-MFMA form
+  ResolvedMatmul d = ResolvedMatmul::from_shapes({64, 1u << 20}, {1u << 20, 64}, {64, 64});
+  d.b_f16 = true;
+  CHECK(w3_group(d) == 0 && !w3_ok(d));
+  // a broadcast A is packed once, whatever the batch
+  d = ResolvedMatmul::from_shapes({1, 8, 4096}, {60000, 4096, 8}, {60000, 8, 8});
+  d.b_f16 = true;
+  CHECK(w3_group(d) == 60000);
+}
+
 int main() {
   test_resolution();
   test_registry();
@@ -393,6 +421,7 @@ int main() {
   test_dtype();
   test_paired_conversion_picks();
   test_packed_a_key();
+  test_w3_scratch();
   std::printf("%d checks, %d failed\n", g_pass + g_fail, g_fail);
   if (g_fail == 0)
     std::printf("all passed\n");

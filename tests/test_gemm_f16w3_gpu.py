@@ -41,6 +41,26 @@ def test_f16w3_shapes(ta, ex, oracle, bt, ba, m, n, k):
             check_f32(ex.download(c), oracle.reference_gemm(ha, hb, bt, m, n, k, **ref), k, oracle)
 
 
+@pytest.mark.parametrize("bb", [400, 1])
+def test_f16w3_batch_in_groups(ta, ex, oracle, bb):
+    """400 planes of one row whose packed A's (300 MiB in all) pass the
+    scratch cap: groups of planes, with a bias and a D of every plane."""
+    bt, m, n, k = 400, 1, 8, 4096
+    ha, hb = oracle.fill_det(bt * m * k, 35), weights(oracle, bb * k * n, 36)
+    hbias, hd = oracle.fill_det(bt * n, 37), oracle.fill_det(bt * m * n, 38)
+    hc = oracle.fill_det(bt * m * n, 39)
+    a, b = ex.tensor_from(ha, shape=[bt, m, k]), ex.tensor_from(hb, shape=[bb, k, n], f16=True)
+    d, bias, c = (ex.tensor_from(hd, shape=[bt, m, n]), ex.tensor_from(hbias, shape=[bt, n]),
+                  ex.tensor_from(hc, shape=[bt, m, n]))
+    ex.run_ops([ta.MatmulOp(a, b, c, accumulate=True, epilogue=ta.Epilogue(
+        bias=bias, activation=ta.ACTIVATION_RELU, binary=ta.BINARY_ADD_SCALED, d=d, beta=0.5))])
+    a64, b64 = ha.reshape(bt, m, k).astype(np.float64), hb.reshape(bb, k, n).astype(np.float64)
+    want = np.maximum(a64 @ b64 + hc.reshape(bt, m, n) + hbias.reshape(bt, 1, n), 0) + 0.5 * hd.reshape(bt, m, n)
+    # f32 sums of K products in any order
+    tol = k * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)) + 1e-6
+    assert np.all(np.abs(ex.download(c).astype(np.float64).reshape(want.shape) - want) <= tol)
+
+
 def test_f16w3_accumulates(ta, ex, oracle):
     m, n, k = 20, 96, 500
     ha, hb, hc = oracle.fill_det(m * k, 41), weights(oracle, k * n, 42), oracle.fill_det(m * n, 43)
