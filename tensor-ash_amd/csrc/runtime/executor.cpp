@@ -30,6 +30,11 @@ namespace {
 
 uint32_t div_ceil(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
+// A scratch block that could not be had.
+struct OutOfScratch : Error {
+  using Error::Error;
+};
+
 // Device scratch owned by a slot or by a prepared graph.  Ops of one
 // submission run in stream order, so they can share one region.
 struct Scratch {
@@ -70,31 +75,22 @@ struct Scratch {
     counters = barrier = nullptr;
     splitk_bytes = partial_bytes = counters_len = mlp_bytes = shadow_bytes = 0;
   }
+  // Grow to at least the given sizes.  A block that is too small is freed
+  // first and its size forgotten with it, so a failed allocation leaves no
+  // size without memory behind.
   void ensure_barrier(bool want) {
     if (!want || barrier)
       return;
-    hip_check(device_malloc(reinterpret_cast<void **>(&barrier), 2 * TA_GEMV_COUNTER_STRIDE * 4),
-              "hipMalloc (GEMV chain barrier)");
+    barrier = static_cast<uint32_t *>(
+        scratch_malloc(2 * TA_GEMV_COUNTER_STRIDE * 4, "hipMalloc (GEMV chain barrier)"));
     hip_check(hipMemset(barrier, 0, 2 * TA_GEMV_COUNTER_STRIDE * 4), "hipMemset (GEMV chain barrier)");
   }
   void ensure_shadow(uint64_t bytes) {
-    if (bytes <= shadow_bytes)
-      return;
-    if (shadow)
-      hip_check(hipFree(shadow), "hipFree");
-    shadow = nullptr;
-    hip_check(device_malloc(&shadow, bytes), "hipMalloc (f16 output copy)");
-    shadow_bytes = bytes;
+    grow(shadow, shadow_bytes, bytes, 1, "hipMalloc (f16 output copy)");
   }
   void ensure_mlp(uint64_t bytes) {
-    if (bytes <= mlp_bytes)
-      return;
-    if (mlp)
-      hip_check(hipFree(mlp), "hipFree");
-    mlp = nullptr;
-    hip_check(device_malloc(&mlp, bytes), "hipMalloc (decode-MLP scratch)");
-    mlp_bytes = bytes;
-    reset_mlp();
+    if (grow(mlp, mlp_bytes, bytes, 1, "hipMalloc (decode-MLP scratch)"))
+      reset_mlp();
   }
   // Zeroed again after a launch that gave up waiting (its hand-off words
   // may carry the generation the next launch would use).
@@ -102,32 +98,42 @@ struct Scratch {
     if (mlp)
       hip_check(hipMemset(mlp, 0, mlp_bytes), "hipMemset (decode-MLP scratch)");
   }
-  // Grow to at least the given sizes.  Counters start at zero (the GEMV
-  // kernels reset them themselves after use).
+  // Counters start at zero (the GEMV kernels reset them themselves after
+  // use).
   void ensure(uint64_t sk_bytes, uint64_t part_bytes, uint64_t n_counters) {
-    if (sk_bytes > splitk_bytes) {
-      if (splitk)
-        hip_check(hipFree(splitk), "hipFree");
-      splitk = nullptr;
-      hip_check(device_malloc(&splitk, sk_bytes), "hipMalloc (split-K scratch)");
-      splitk_bytes = sk_bytes;
+    grow(splitk, splitk_bytes, sk_bytes, 1, "hipMalloc (split-K scratch)");
+    grow(partial, partial_bytes, part_bytes, 1, "hipMalloc (GEMV partials)");
+    if (grow(counters, counters_len, n_counters, 4, "hipMalloc (GEMV counters)"))
+      hip_check(hipMemset(counters, 0, counters_len * 4), "hipMemset (GEMV counters)");
+  }
+
+private:
+  // TA_SCRATCH_LIMIT (bytes) refuses larger blocks as if memory were out.
+  static void *scratch_malloc(uint64_t bytes, const char *what) {
+    const char *limit = std::getenv("TA_SCRATCH_LIMIT");
+    void *p = nullptr;
+    const hipError_t err = limit && bytes > std::strtoull(limit, nullptr, 10)
+                               ? hipErrorOutOfMemory
+                               : device_malloc(&p, bytes);
+    if (err == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      throw OutOfScratch(std::string(what) + " failed: " + hipGetErrorString(err));
     }
-    if (part_bytes > partial_bytes) {
-      if (partial)
-        hip_check(hipFree(partial), "hipFree");
-      partial = nullptr;
-      hip_check(device_malloc(&partial, part_bytes), "hipMalloc (GEMV partials)");
-      partial_bytes = part_bytes;
-    }
-    if (n_counters > counters_len) {
-      if (counters)
-        hip_check(hipFree(counters), "hipFree");
-      counters = nullptr;
-      hip_check(device_malloc(reinterpret_cast<void **>(&counters), n_counters * 4),
-                "hipMalloc (GEMV counters)");
-      hip_check(hipMemset(counters, 0, n_counters * 4), "hipMemset (GEMV counters)");
-      counters_len = n_counters;
-    }
+    hip_check(err, what);
+    return p;
+  }
+  template <class T>
+  static bool grow(T *&block, uint64_t &size, uint64_t want, uint64_t unit, const char *what) {
+    if (want <= size)
+      return false;
+    T *old = block;
+    block = nullptr;
+    size = 0;
+    if (old)
+      hip_check(hipFree(old), "hipFree");
+    block = static_cast<T *>(scratch_malloc(want * unit, what));
+    size = want;
+    return true;
   }
 };
 
@@ -203,7 +209,23 @@ struct OpPlan {
   bool w3 = false;
   uint32_t mlp_layers = 0;
   uint32_t chain_jobs = 0;
+
+  // Back to the kernel's FP32-MFMA form, which needs no scratch; false when
+  // the op has no other form.
+  bool leave_split_products() {
+    const bool any = x6 || w3;
+    x6 = 0;
+    w3 = false;
+    return any;
+  }
 };
+
+bool leave_split_products(std::vector<OpPlan> &plans) {
+  bool any = false;
+  for (OpPlan &p : plans)
+    any = p.leave_split_products() || any;
+  return any;
+}
 
 struct ScratchNeed {
   uint64_t splitk = 0, partial = 0, counters = 0, mlp = 0, shadow = 0;
@@ -1050,6 +1072,25 @@ struct ExecutorImpl {
     }
   }
 
+  static void ensure(Scratch &sc, const ScratchNeed &need) {
+    sc.ensure(need.splitk, need.partial, need.counters);
+    sc.ensure_mlp(need.mlp);
+    sc.ensure_shadow(need.shadow);
+    sc.ensure_barrier(need.barrier);
+  }
+  // Scratch for the plans.  Split products need room that their FP32-MFMA
+  // forms do not: where it cannot be had, the ops run in those.
+  void reserve(Scratch &sc, const std::vector<ResolvedMatmul> &res,
+               std::vector<OpPlan> &plans) const {
+    try {
+      ensure(sc, total_need(res, plans));
+    } catch (const OutOfScratch &) {
+      if (!leave_split_products(plans))
+        throw;
+      ensure(sc, total_need(res, plans));
+    }
+  }
+
   ScratchNeed total_need(const std::vector<ResolvedMatmul> &res,
                          const std::vector<OpPlan> &plans) const {
     ScratchNeed need;
@@ -1467,12 +1508,8 @@ struct ExecutorImpl {
   // Submit `ops` on a slot and wait; returns GPU ns between the events.
   uint64_t submit_and_wait(Slot *slot, const std::vector<MatmulOp> &ops,
                            const std::vector<ResolvedMatmul> &res,
-                           const std::vector<OpPlan> &plans) const {
-    ScratchNeed need = total_need(res, plans);
-    slot->scratch.ensure(need.splitk, need.partial, need.counters);
-    slot->scratch.ensure_mlp(need.mlp);
-    slot->scratch.ensure_shadow(need.shadow);
-    slot->scratch.ensure_barrier(need.barrier);
+                           std::vector<OpPlan> plans) const {
+    reserve(slot->scratch, res, plans);
     return submit_on(slot, ops, res, plans, slot->scratch);
   }
   // run_ops with several independent ops (src/executor/dispatch.rs:55-60:
@@ -1521,12 +1558,7 @@ struct ExecutorImpl {
         parts[l].res.push_back(res[i]);
         parts[l].plans.push_back(plans[i]);
       }
-      const ScratchNeed need = total_need(parts[l].res, parts[l].plans);
-      Scratch &sc = l == 0 ? slot->scratch : slot->side[l - 1].scratch;
-      sc.ensure(need.splitk, need.partial, need.counters);
-      sc.ensure_mlp(need.mlp);
-      sc.ensure_shadow(need.shadow);
-      sc.ensure_barrier(need.barrier);
+      reserve(l == 0 ? slot->scratch : slot->side[l - 1].scratch, parts[l].res, parts[l].plans);
     }
     hip_check(hipEventRecord(slot->start, slot->stream), "hipEventRecord");
     hip_check(hipEventRecord(slot->fork, slot->stream), "hipEventRecord");
@@ -1648,6 +1680,12 @@ struct ExecutorImpl {
         need.merge(total_need(st.res, st.plans));
     return need;
   }
+  static bool exec_leave_split_products(std::vector<ExecStep> &steps) {
+    bool any = false;
+    for (ExecStep &st : steps)
+      any = leave_split_products(st.plans) || any;
+    return any;
+  }
   static bool exec_has_mlp(const std::vector<ExecStep> &steps) {
     for (const ExecStep &st : steps)
       if (st.matmul && has_mlp(st.plans))
@@ -1668,14 +1706,16 @@ struct ExecutorImpl {
       fail("run_exec_ops: empty op list");
     ctx->make_current();
     uint64_t flops = 0;
-    const std::vector<ExecStep> steps = plan_exec(ops, flops);
+    std::vector<ExecStep> steps = plan_exec(ops, flops);
     Lease lease(this);
     Slot *slot = lease.s;
-    const ScratchNeed need = exec_need(steps);
-    slot->scratch.ensure(need.splitk, need.partial, need.counters);
-    slot->scratch.ensure_mlp(need.mlp);
-    slot->scratch.ensure_shadow(need.shadow);
-    slot->scratch.ensure_barrier(need.barrier);
+    try {
+      ensure(slot->scratch, exec_need(steps));
+    } catch (const OutOfScratch &) {
+      if (!exec_leave_split_products(steps))
+        throw;
+      ensure(slot->scratch, exec_need(steps));
+    }
     hip_check(hipEventRecord(slot->start, slot->stream), "hipEventRecord");
     record_exec(steps, slot->scratch, slot->host_status, slot->stream);
     hip_check(hipEventRecord(slot->end, slot->stream), "hipEventRecord");
@@ -1693,10 +1733,16 @@ struct ExecutorImpl {
     ctx->make_current();
     uint64_t flops = 0;
     auto steps = std::make_shared<std::vector<ExecStep>>(plan_exec(ops, flops));
-    return capture(owner, ops.size(), flops, exec_need(*steps), exec_has_mlp(*steps),
-                   [this, steps](Scratch &scratch, uint32_t *status, hipStream_t stream) {
-                     record_exec(*steps, scratch, status, stream);
-                   });
+    auto rec = [this, steps](Scratch &scratch, uint32_t *status, hipStream_t stream) {
+      record_exec(*steps, scratch, status, stream);
+    };
+    try {
+      return capture(owner, ops.size(), flops, exec_need(*steps), exec_has_mlp(*steps), rec);
+    } catch (const OutOfScratch &) { // raised before anything is recorded
+      if (!exec_leave_split_products(*steps))
+        throw;
+      return capture(owner, ops.size(), flops, exec_need(*steps), exec_has_mlp(*steps), rec);
+    }
   }
 
   // ---- tuning (src/executor/tuning.rs) ----
@@ -2043,8 +2089,11 @@ struct ExecutorImpl {
     for (const auto &op : ops)
       res.push_back(ResolvedMatmul::from_op(op));
     const uint64_t flops = total_flops(res);
-    // Data-parallel routes only, like the reference: split-K would need
-    // its scratch baked into the graph for the handle's lifetime.
+    // No split-K routes, like the reference, whose scratch they would have
+    // baked into the graph.  Other scratch (f16 copies, packed pieces of
+    // split products, up to kF32X6ScratchCapBytes) belongs to the handle and
+    // is freed with it; where the pieces cannot be had, the op is recorded
+    // in its FP32-MFMA form.
     std::vector<OpPlan> plans;
     for (size_t i = 0; i < res.size(); ++i)
       plans.push_back(plan_op(ops[i], res[i], false));
@@ -2054,10 +2103,16 @@ struct ExecutorImpl {
     for (size_t i = 0; i < ops.size(); ++i)
       check_supported(KERNEL_SPECS[plans[i].kernel], res[i]);
 
-    return capture(owner, ops.size(), flops, total_need(res, plans), has_mlp(plans),
-                   [&](Scratch &scratch, uint32_t *status, hipStream_t stream) {
-                     record(ops, res, plans, scratch, status, stream);
-                   });
+    auto rec = [&](Scratch &scratch, uint32_t *status, hipStream_t stream) {
+      record(ops, res, plans, scratch, status, stream);
+    };
+    try {
+      return capture(owner, ops.size(), flops, total_need(res, plans), has_mlp(plans), rec);
+    } catch (const OutOfScratch &) { // raised before anything is recorded
+      if (!leave_split_products(plans))
+        throw;
+      return capture(owner, ops.size(), flops, total_need(res, plans), has_mlp(plans), rec);
+    }
   }
 
   // Record once into a hipGraph on a private stream, with graph-owned
@@ -2078,10 +2133,12 @@ struct ExecutorImpl {
     hip_check(hipEventCreate(&e1), "hipEventCreate");
     p->ev_end_ = e1;
     Scratch scratch;
-    scratch.ensure(need.splitk, need.partial, need.counters);
-    scratch.ensure_mlp(need.mlp);
-    scratch.ensure_shadow(need.shadow);
-    scratch.ensure_barrier(need.barrier);
+    try {
+      ensure(scratch, need);
+    } catch (...) {
+      scratch.release();
+      throw;
+    }
     p->scratch_ = {scratch.splitk, scratch.partial, scratch.counters, scratch.mlp, scratch.shadow,
                    scratch.barrier};
     p->mlp_scratch_ = scratch.mlp;
