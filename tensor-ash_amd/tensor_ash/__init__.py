@@ -390,7 +390,8 @@ def _ops_array(ops: Sequence[MatmulOp]):
             pack(buf, i * size, o.a.handle, o.b.handle, o.c.handle, o.alpha, int(o.accumulate),
                  bias.handle if bias is not None and bias else 0, e.activation, e.binary,
                  d.handle if d is not None and d else 0, e.beta, packed)
-    except struct.error:  # no handle (a closed tensor: the C call reports the null), or no plain number
+    # no handle (a closed tensor: the C call reports the null), no plain number, or a scale past f32 (ctypes: inf)
+    except (struct.error, OverflowError):
         if any(o.normed_a is not None or o.store is not None for o in ops):
             return (_OpV3 * n)(*[o._raw_v3() for o in ops]), 3
         if any(o.packed_b for o in ops):

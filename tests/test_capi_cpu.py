@@ -159,3 +159,23 @@ def test_ops_array_packs_what_the_structures_hold(ta):
         for a, op in zip(arr, ops):
             want = {1: op._raw, 2: lambda: ta._OpV2(op._raw(), int(op.packed_b)), 3: op._raw_v3}[version]()
             assert ctypes.string_at(ctypes.byref(a), ctypes.sizeof(a)) == bytes(want)
+
+
+@pytest.mark.parametrize("alpha,beta", [(1e39, 0.0), (-1e39, 1.0), (1.0, 1e300), (np.float64(-3.5e38), -4e38)])
+def test_ops_array_takes_scales_past_f32(ta, alpha, beta):
+    """alpha and beta beyond the largest f32 become infinities, as the
+    structures built field by field hold them, in every version."""
+    import ctypes
+
+    class T:
+        handle = 0x7F0000001000
+
+    t = T()
+    op = dict(alpha=alpha, epilogue=ta.Epilogue(None, 0, 1, t, beta))
+    plain = ta.MatmulOp(t, t, t)
+    for ops in ([ta.MatmulOp(t, t, t, **op)], [plain, ta.MatmulOp(t, t, t, packed_b=True, **op)],
+                [ta.MatmulOp(t, t, t, **op), ta.MatmulOp(t, t, t, normed_a=(t, 1e-5))]):
+        arr, version = ta._ops_array(ops)
+        for a, o in zip(arr, ops):
+            want = {1: o._raw, 2: lambda: ta._OpV2(o._raw(), int(o.packed_b)), 3: o._raw_v3}[version]()
+            assert ctypes.string_at(ctypes.byref(a), ctypes.sizeof(a)) == bytes(want)
