@@ -7,8 +7,8 @@
 // bf16 pieces (8 + 3 bits, exact), and of the six piece products the five
 // largest are summed on v_mfma_f32_32x32x16_bf16; the sixth is below 2^-27
 // of the product.  A result that is not finite (an infinite operand meets
-// zero pieces), or a row whose values are all below 2^-95, makes its tile
-// compute whole f32 products instead.
+// zero pieces), or a row with a value that is not exactly its three pieces
+// (nonzero below 2^-110), makes its tile compute whole f32 products instead.
 //
 // Split.  A workgroup owns 32 or 64 rows x 64 columns and a run of 64-deep K
 // stages; several share a tile's K so that two workgroups per CU stream
@@ -143,7 +143,7 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
         commit(s);
       }
 
-    // Rows whose values are all tiny (while the first stages load).
+    // Rows that are not exactly their pieces (while the first stages load).
     bool whole = false;
     for (uint32_t r = tid; r < (uint32_t)BM; r += T) {
       const uint32_t rows = q.blocks_a * 32u;
@@ -151,7 +151,7 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
       uint32_t bits = 0;
       for (uint32_t c = 0; c < q.chunks; ++c)
         bits |= from[(uint64_t)c * rows];
-      whole = whole || (bits != 0u && (bits & 0x70000000u) == 0u);
+      whole = whole || bits != 0u;
     }
 
     uint32_t st = 0;

@@ -7,20 +7,19 @@
 // the nine piece products the six largest are summed:
 //   hi hi, hi mid, mid hi, mid mid, hi lo, lo hi.
 // The three left out are at most 2^-26 |a b| together, a quarter of the
-// rounding of one f32 product.  Measured against f64 (normal inputs): K =
+// rounding of one f32 product: a single product is thus off by up to 1.25
+// times that rounding.  Measured against f64 (normal inputs): K =
 // 4096 9.0e-7 (256 x 256 tile) and 5.1e-7 (128 x 128), against 1.1e-6 of the
 // FP32 MFMAs; K = 777 2e-7 against 5e-7.  Ceiling: a sixth of the bf16 rate.
 //
-// bf16 has f32's exponent range, so no scaling is needed, with three
-// exceptions, in which a tile is computed on the FP32 MFMAs (GemmF32) in
-// the same launch:
-//  * a row of A or column of B whose values are all below 2^-95: the low
-//    pieces of values below 2^-110 would be rounded to bf16's smallest
-//    denormal, which matters only if nothing larger shares their sums.  The
-//    pack leaves the OR of each row's bits, from which a workgroup reads
-//    whether any exponent of its rows reaches 32 (biased);
-//  * an infinity or NaN (its lower pieces are NaN), and values that round
-//    past the largest bf16: the accumulators come out non-finite.
+// bf16 has f32's exponent range, so no scaling is needed.  Values that are
+// not exactly their three pieces (nonzero below 2^-110, where the lowest bits
+// fall under bf16's smallest denormal; past the largest bf16; infinities and
+// NaN, whose lower pieces are NaN) send their tiles to the FP32 MFMAs
+// (GemmF32) in the same launch: the pack leaves a word per row and column that
+// says whether any of its values is one, and a sum that comes out non-finite
+// says the same.  Such a tile costs both forms.  Denormals are kept throughout
+// by the conversions and the MFMAs.
 #include "gemm_f32_tile.h"
 #include "split3.h"
 
@@ -91,8 +90,8 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
       if (s < (int)kts)
         issue(s);
 
-    // Rows and columns whose values are all tiny (while the first stages load).
-    bool tiny = false;
+    // Rows and columns that are not exactly their pieces (while the first stages load).
+    bool inexact = false;
     {
       const uint32_t ra = q.blocks_a * 32u, rb = q.blocks_b * 32u;
       const uint32_t *ba = q.bits_a + (q.plane_a ? (uint64_t)batch * q.chunks * ra : 0) + tm * BM;
@@ -103,7 +102,7 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
         uint32_t bits = 0;
         for (uint32_t c = 0; c < q.chunks; ++c)
           bits |= from[(uint64_t)c * step];
-        tiny = tiny || (bits != 0u && (bits & 0x70000000u) == 0u);
+        inexact = inexact || bits != 0u;
       }
     }
 
@@ -180,7 +179,7 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
               acc[f / FN][f % FN][r] += red[(((k - 1) * WT + w2) * FM * FN + f) * 1024 + r * 64 + lane];
       }
     }
-    bool whole = tiny;
+    bool whole = inexact;
     if (kg == 0) {
 #pragma unroll
       for (int f = 0; f < FM; ++f)

@@ -94,7 +94,8 @@ typedef struct GemmArgs {
 // block and k-step; blocks and k-steps past the matrix are zeros.
 #define TA_X6_STEP_BYTES 3072u
 // k-steps one workgroup of the pack covers (4 waves x 4 steps); it leaves
-// one word per row / column of its block: the OR of its values' bits.
+// one word per row / column of its block, zero if every value is exactly the
+// sum of its three pieces.
 #define TA_X6_CHUNK_STEPS 16u
 
 typedef struct PackX3Job {

@@ -8,8 +8,12 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// x = out[0] + ... + out[P - 1] (P = 3: exactly), each rounded to nearest.
-template <int P> TA_DEVICE void split_bf16(const float (&x)[8], bf16x8 (&out)[P]) {
+// x = out[0] + ... + out[P - 1] + what is left over, each piece rounded to
+// nearest.  P = 3 leaves nothing from 2^-110 up to the largest bf16, whose
+// lowest bits end at bf16's smallest denormal (smaller values leave nothing
+// when their lower bits are zeros; infinities and NaN leave NaN).  Returns
+// the OR of the eight remainders' bits: zero if all are +0.
+template <int P> TA_DEVICE uint32_t split_bf16(const float (&x)[8], bf16x8 (&out)[P]) {
   float r[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
@@ -26,6 +30,11 @@ template <int P> TA_DEVICE void split_bf16(const float (&x)[8], bf16x8 (&out)[P]
       r[i] -= __uint_as_float(w << 16);
       r[i + 1] -= __uint_as_float(w & 0xffff0000u);
     }
+  uint32_t left = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    left |= __float_as_uint(r[i]);
+  return left;
 }
 
 // One workgroup of a pack job: four waves of 4 k-steps each.  ROWS: A's 32
@@ -74,12 +83,9 @@ template <bool ROWS> TA_DEVICE void pack_job(const PackX3Job &p, uint32_t group,
     for (int i = 0; i < 4; ++i) {
       const uint32_t step = step0 + (ROWS ? i : trip * 2 + i / 2);
       const uint32_t half = ROWS ? lane >> 5 : i % 2;
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        bits |= __float_as_uint(x[i][e]);
-      if (step < p.ksteps) {
+      if (step < p.ksteps) { // zeros past it
         bf16x8 o[3];
-        split_bf16(x[i], o);
+        bits |= split_bf16(x[i], o);
 #pragma unroll
         for (int q = 0; q < 3; ++q)
           dst[((uint64_t)step * 3u + q) * 64u + half * 32u + (lane & 31u)] = o[q];
@@ -97,7 +103,7 @@ template <bool ROWS> TA_DEVICE void pack_job(const PackX3Job &p, uint32_t group,
       if (lane >= 32u)
         return;
     }
-    p.bits[((uint64_t)plane * p.chunks + chunk) * p.blocks * 32u + row] = bits & 0x7fffffffu;
+    p.bits[((uint64_t)plane * p.chunks + chunk) * p.blocks * 32u + row] = bits;
   }
 }
 

@@ -124,3 +124,19 @@ def test_f16w3_special_values(ta, ex, n):
     assert np.array_equal(got[inf], exact[inf].astype(np.float32))
     fine = np.isfinite(exact)
     assert np.max(np.abs(got[fine] - exact[fine]) / exact[fine]) <= k * 2.0 ** -24
+
+
+@pytest.mark.parametrize("small", [-109, -111, -115, -125, -140])
+def test_f16w3_small_values_beside_large_ones(ta, ex, small):
+    """Values of A too small for three whole pieces, in rows that also hold
+    large ones, which meet zero weights: each result is one product by a
+    power of two, exact in f32."""
+    rng = np.random.default_rng(9)
+    m, n, k = 40, 72, 200
+    a, b = np.zeros((m, k), np.float32), np.zeros((k, n), np.float32)
+    tiny = np.ldexp(rng.uniform(1, 2, m).astype(np.float32), small).astype(np.float32)
+    a[:, 0], a[:, 77], b[77] = rng.uniform(1, 2, m), tiny, 2.0 ** 15
+    c = ex.tensor([m, n])
+    ex.run_ops([ta.MatmulOp(ex.tensor_from(a), ex.tensor_from(b, f16=True), c)])
+    want = tiny[:, None].astype(np.float64) * 2.0 ** 15 * np.ones(n)
+    assert np.array_equal(ex.download(c), want.astype(np.float32))

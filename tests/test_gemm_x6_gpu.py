@@ -70,7 +70,7 @@ def test_x6_special_values(ta, ex, monkeypatch, tile):
     m, n, k = 200, 150, 96
     a, b = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32), rng.uniform(0.5, 1.5, (k, n)).astype(np.float32)
     a[3, 5], a[70, 1], a[150, 9] = np.inf, np.nan, np.float32(3.402e38)
-    a[100] *= np.float32(2.0 ** -112)  # every value below 2^-95
+    a[100] *= np.float32(2.0 ** -112)  # too small for three whole pieces
     b[7, 33] = -np.inf
     got = product(ta, ex, a, b, monkeypatch, tile)
     with np.errstate(all="ignore"):
@@ -86,6 +86,44 @@ def test_x6_special_values(ta, ex, monkeypatch, tile):
     big = np.isfinite(exact) & (np.abs(exact) > 3.5e38)
     assert np.all(np.isposinf(got[big])) and np.any(big)
     assert np.max(np.abs(got[fine] - exact[fine]) / np.abs(exact[fine])) <= 2 * k * 2.0 ** -24
+
+
+def mantissas(rng, *shape):
+    return rng.uniform(1, 2, shape).astype(np.float32)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("side", ["a", "b"])
+@pytest.mark.parametrize("small", [-109, -111, -115, -125, -140])
+def test_x6_small_values_beside_large_ones(ta, ex, monkeypatch, tile, side, small):
+    """Values too small for three whole pieces, in rows or columns that also
+    hold large ones, where the other operand has zeros against the large
+    ones: each result is one product by a power of two, exact in f32."""
+    rng = np.random.default_rng(9)
+    m, n, k = 130, 70, 40
+    a, b = np.zeros((m, k), np.float32), np.zeros((k, n), np.float32)
+    tiny = np.ldexp(mantissas(rng, m if side == "a" else n), small).astype(np.float32)  # denormals too
+    if side == "a":
+        a[:, 0], a[:, 17], b[17] = mantissas(rng, m), tiny, np.float32(2.0 ** 100)
+        want = tiny[:, None].astype(np.float64) * 2.0 ** 100 * np.ones(n)
+    else:
+        b[0], b[17], a[:, 17] = mantissas(rng, n), tiny, np.float32(2.0 ** 100)
+        want = tiny[None, :].astype(np.float64) * 2.0 ** 100 * np.ones((m, 1))
+    assert np.array_equal(product(ta, ex, a, b, monkeypatch, tile), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("ea,eb", [(-100, 0), (-60, -62), (-70, -70), (-30, -105)])
+def test_x6_small_results(ta, ex, monkeypatch, tile, ea, eb):
+    """Whole pieces whose products are near f32's smallest normal: f32 sums
+    of K products in any order, and the rounding of denormals."""
+    rng = np.random.default_rng(10)
+    m, n, k = 100, 90, 48
+    a, b = np.ldexp(mantissas(rng, m, k), ea).astype(np.float32), np.ldexp(mantissas(rng, k, n), eb).astype(np.float32)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    got = product(ta, ex, a, b, monkeypatch, tile).astype(np.float64)
+    # six piece products of each pair round to multiples of 2^-149
+    assert np.all(np.abs(got - exact) <= k * (2.0 ** -24 * exact + 6 * 2.0 ** -150))
 
 
 def test_x6_in_graphs_and_prepared(ta, ex, oracle, monkeypatch):
