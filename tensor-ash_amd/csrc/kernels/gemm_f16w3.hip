@@ -19,6 +19,11 @@
 // take turns (four waves on 128-column tiles, one workgroup per CU: 53 us
 // against 41 below).  B is staged as it lies in memory and reaches the
 // matrix cores through ds_read_b64_tr_b16; A's pieces are whole KiB.
+// Whole f32 products (see above) run on the FP32 MFMAs from operands as they
+// lie in memory: every workgroup over its own stages where A's words say so
+// before the second stage, the last one over all of K where a sum comes out
+// non-finite.  With such a value in every row: 16 x 4096 x 14336 104 us, 24 x
+// 3648 x 2816 42 (a dot product per thread: 6800 and 2010).
 //
 // Kernel time: 16 x 4096 x 14336 41 us = 2.9 TB/s (FP32-MFMA tiles without
 // split-K: 1140 us), 24 x 3648 x 2816 17.5 us (217); each op adds a 5 us pack
@@ -50,7 +55,8 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
   static TA_DEVICE void run(const GemmW3Args &q) {
     const GemmArgs &p = q.g;
     __shared__ __attribute__((aligned(1024))) char smem[SMEM];
-    __shared__ uint32_t last_flag;
+    constexpr int RW = (BM + 63) / 64;
+    __shared__ uint32_t last_flag, whole_sh[RW];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t kg = wave >> 1, wn = wave & 1u;
@@ -143,7 +149,8 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
         commit(s);
       }
 
-    // Rows that are not exactly their pieces (while the first stages load).
+    // Rows that are not exactly their pieces (while the first stages load):
+    // every workgroup of the tile reads the same words and takes whole values.
     bool whole = false;
     for (uint32_t r = tid; r < (uint32_t)BM; r += T) {
       const uint32_t rows = q.blocks_a * 32u;
@@ -153,6 +160,11 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
         bits |= from[(uint64_t)c * rows];
       whole = whole || bits != 0u;
     }
+    // (the words of the waves that hold rows are read after the first stage's
+    // barrier)
+    whole = __any(whole);
+    if (wave < RW && lane == 0)
+      whole_sh[wave] = whole;
 
     uint32_t st = 0;
     for (uint32_t kt = 0; kt < kts; ++kt) {
@@ -164,6 +176,15 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
       } else
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads(); // stage kt landed; every wave is done with stage kt - 1
+      if (kt == 0) {
+        uint32_t any = 0;
+#pragma unroll
+        for (int w = 0; w < RW; ++w)
+          any |= whole_sh[w];
+        whole = __builtin_amdgcn_readfirstlane(any) != 0u;
+        if (whole)
+          break;
+      }
       const uint32_t ahead = st + AHEAD < NS ? st + AHEAD : st + AHEAD - NS;
       if (kt + AHEAD < kts)
         issue(kt + AHEAD, ahead);
@@ -211,26 +232,66 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
     for (int i = 0; i < NB; ++i)
       sum[i] = acc[i / FN][i % FN] + acc2[i / FN][i % FN];
 
-    // The k-step groups meet in LDS, in group order; waves 0 and 1 go on.
-    float *red = reinterpret_cast<float *>(smem);
-    __syncthreads();
-    if (kg > 0) {
+    // This wave's part of stages [from, to) in whole f32 products, with A and
+    // B as they lie in memory (lane half h takes k = 8 h .. 8 h + 7 of a step).
+    const uint32_t lr = lane & 31u, lg = lane >> 5;
+    auto whole_stages = [&](uint32_t from, uint32_t to) __attribute__((always_inline)) {
+      const float *Af = static_cast<const float *>(p.a) + (uint64_t)batch * p.stride_a;
 #pragma unroll
       for (int i = 0; i < NB; ++i)
+        sum[i] = f32x16{};
+#pragma unroll 2
+      for (uint32_t stage = from; stage < to; ++stage) {
+        const uint32_t k0 = stage * (uint32_t)BK + kg * 16u + lg * 8u;
+        float a[FM][8], b[FN][8];
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          red[(((kg - 1) * 2 + wn) * NB + i) * 1024 + r * 64 + lane] = sum[i][r];
-    }
-    __syncthreads();
-    if (kg == 0) {
+        for (uint32_t e = 0; e < 8u; ++e) {
+          const uint32_t k = min(k0 + e, p.k - 1u);
+          const bool in = k0 + e < p.k;
 #pragma unroll
-      for (int k = 1; k < KG; ++k)
+          for (int f = 0; f < FM; ++f) {
+            const float v = Af[(uint64_t)min(m0 + f * 32u + lr, p.m - 1u) * p.k + k];
+            a[f][e] = in ? v : 0.0f;
+          }
+#pragma unroll
+          for (int x = 0; x < FN; ++x) {
+            const float v = (float)B[(uint64_t)k * p.n + min(n0 + (wn * FN + x) * 32u + lr, p.n - 1u)];
+            b[x][e] = in ? v : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+            sum[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i / FN][e], b[i % FN][e], sum[i], 0, 0, 0);
+      }
+    };
+    // The k-step groups meet in LDS, in group order; waves 0 and 1 go on.
+    float *red = reinterpret_cast<float *>(smem);
+    auto meet = [&]() __attribute__((always_inline)) {
+      if (kg > 0) {
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            sum[i][r] += red[(((k - 1) * 2 + wn) * NB + i) * 1024 + r * 64 + lane];
-    }
+            red[(((kg - 1) * 2 + wn) * NB + i) * 1024 + r * 64 + lane] = sum[i][r];
+      }
+      __syncthreads();
+      if (kg == 0) {
+#pragma unroll
+        for (int k = 1; k < KG; ++k)
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              sum[i][r] += red[(((k - 1) * 2 + wn) * NB + i) * 1024 + r * 64 + lane];
+      }
+    };
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // loads of a loop that was left
+    if (whole)
+      whole_stages(slo, slo + kts);
+    __syncthreads(); // every wave is done with the stages' LDS
+    meet();
     if (S > 1) {
       const uint64_t tile_id = (uint64_t)batch * p.tiles_m * p.tiles_n + blockIdx.x;
       constexpr uint32_t SLOT = NB * 16 * 128; // words of one partial tile
@@ -287,26 +348,21 @@ template <int FM, int NS, bool ALIGNED> struct GemmW3 {
     // (l / 32) + r % 4.
     auto row_of = [&](int i, int r) { return m0 + (i / FN) * 32u + 8u * (r / 4) + 4u * (lane >> 5) + (r % 4); };
     auto col_of = [&](int i) { return n0 + (wn * FN + i % FN) * 32u + (lane & 31u); };
-    if (kg == 0) {
+    // An infinite weight or a sum past f32: this workgroup computes the tile
+    // again, over all of K.
+    if (!whole) {
+      bool wrong = false;
+      if (kg == 0) {
 #pragma unroll
-      for (int i = 0; i < NB; ++i)
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          whole = whole || (row_of(i, r) < p.m && col_of(i) < p.n && !__builtin_isfinite(sum[i][r]));
-    }
-    if (__syncthreads_or(whole)) {
-      const float *Af = static_cast<const float *>(p.a) + (uint64_t)batch * p.stride_a;
-      const uint32_t col = n0 + tid % BN;
-      for (uint32_t row = m0 + tid / BN; row < min(m0 + (uint32_t)BM, p.m); row += T / BN) {
-        float v = 0.0f;
-        if (col < p.n) {
-          for (uint32_t k = 0; k < p.k; ++k)
-            v = fmaf(Af[(uint64_t)row * p.k + k], (float)B[(uint64_t)k * p.n + col], v);
-          const uint64_t at = (uint64_t)batch * p.stride_c + (uint64_t)row * p.n + col;
-          p.c[at] = ta_epilogue(v, p, at, col, batch);
-        }
+          for (int r = 0; r < 16; ++r)
+            wrong = wrong || (row_of(i, r) < p.m && col_of(i) < p.n && !__builtin_isfinite(sum[i][r]));
       }
-      return;
+      if (__syncthreads_or(wrong)) {
+        whole_stages(0, steps);
+        meet();
+      }
     }
     if (kg == 0) {
 #pragma unroll

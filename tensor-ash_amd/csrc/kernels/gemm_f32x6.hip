@@ -18,8 +18,11 @@
 // NaN, whose lower pieces are NaN) send their tiles to the FP32 MFMAs
 // (GemmF32) in the same launch: the pack leaves a word per row and column that
 // says whether any of its values is one, and a sum that comes out non-finite
-// says the same.  Such a tile costs both forms.  Denormals are kept throughout
-// by the conversions and the MFMAs.
+// says the same.  A tile of the first kind leaves before its second stage, one
+// of the second costs both forms.  With a value of the first kind in every row:
+// 4096^3 1414 us, 2048^3 196, 1000^3 91 (split products 770, 104, 32; FP32
+// MFMA 965, 188, 50, whose kernel picks its own tile).  Denormals are kept
+// throughout by the conversions and the MFMAs.
 #include "gemm_f32_tile.h"
 #include "split3.h"
 
@@ -55,6 +58,7 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
   static TA_DEVICE void run(const GemmX6Args &q) {
     const GemmArgs &p = q.g;
     __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+    __shared__ uint32_t inexact_sh[W];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t kg = wave / WT, w2 = wave % WT, wm = w2 / WGN, wn = w2 % WGN;
@@ -105,6 +109,10 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
         inexact = inexact || bits != 0u;
       }
     }
+    // (one word per wave, read after the first stage's barrier)
+    inexact = __any(inexact);
+    if (lane == 0)
+      inexact_sh[wave] = inexact;
 
     f32x16 acc[FM][FN], acc2[TWO ? FM : 1][TWO ? FN : 1];
 #pragma unroll
@@ -122,6 +130,15 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
       else
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads(); // stage kt landed; every wave is done with stage kt - 1
+      if (kt == 0) {
+        uint32_t any = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+          any |= inexact_sh[w];
+        inexact = __builtin_amdgcn_readfirstlane(any) != 0u;
+        if (inexact)
+          break;
+      }
       if (kt + NS - 1 < kts)
         issue(nst);
       const uint32_t ab = lds0 + st * STAGE + lo + wm * FM * (G * STEP) + kg * STEP;
@@ -158,6 +175,7 @@ template <int BM, int BN, int WGM, int WGN, int G, int NS, bool TWO> struct Gemm
           for (int r = 0; r < 16; ++r)
             acc[f][g][r] += acc2[f][g][r];
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // loads of a loop that was left
     __syncthreads();
     if constexpr (G > 1) {
       float *red = reinterpret_cast<float *>(smem);

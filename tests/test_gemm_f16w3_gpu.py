@@ -140,3 +140,38 @@ def test_f16w3_small_values_beside_large_ones(ta, ex, small):
     ex.run_ops([ta.MatmulOp(ex.tensor_from(a), ex.tensor_from(b, f16=True), c)])
     want = tiny[:, None].astype(np.float64) * 2.0 ** 15 * np.ones(n)
     assert np.array_equal(ex.download(c), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("bt,m,n,k", [(1, 33, 65, 1000), (1, 63, 136, 161), (1, 9, 8, 4096), (3, 8, 130, 513), (2, 40, 72, 2800)])
+@pytest.mark.parametrize("special", ["a", "b"])
+def test_f16w3_whole_f32_tiles(ta, ex, oracle, bt, m, n, k, special):
+    """The form for values that do not split, at edges of rows, columns and K
+    windows, with every epilogue operand: a small value in each plane of A,
+    or an infinite weight in a column of its own."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((bt, m, k)).astype(np.float32)
+    b = (rng.standard_normal((bt, k, n)) * 0.5).astype(np.float16).astype(np.float32)
+    col = np.zeros(n, bool)
+    if special == "a":
+        a[:, m // 2, k - 1] = 1e-37
+    else:
+        b[:, k - 1, n - 1] = np.inf
+        col[n - 1] = True
+    shape = [m, n] if bt == 1 else [bt, m, n]
+    bias, d, old = rng.standard_normal((bt, n)), rng.standard_normal((bt, m, n)), rng.standard_normal((bt, m, n))
+    bias, d, old = (x.astype(np.float32) for x in (bias, d, old))
+    ta_ = ex.tensor_from(a if bt > 1 else a[0])
+    tb = ex.tensor_from(b if bt > 1 else b[0], f16=True)
+    tbias, td, c = (ex.tensor_from(bias.reshape(-1)[:n] if bt == 1 else bias), ex.tensor_from(d.reshape(shape)),
+                    ex.tensor_from(old.reshape(shape)))
+    for _ in range(2):  # the split counters are back at zero
+        ex.upload(c, old.reshape(-1))
+        ex.run_ops([ta.MatmulOp(ta_, tb, c, alpha=0.5, accumulate=True, epilogue=ta.Epilogue(
+            bias=tbias, binary=ta.BINARY_MUL, d=td))])
+        got = ex.download(c).reshape(bt, m, n).astype(np.float64)
+        with np.errstate(all="ignore"):
+            a64, b64 = a.astype(np.float64), b.astype(np.float64)
+            want = (0.5 * (a64 @ b64) + old + bias[:, None, :]) * d
+            tol = k * 2.0 ** -24 * ((np.abs(a64) @ np.abs(b64)) + np.abs(old) + np.abs(bias[:, None, :]) + 1) * np.abs(d)
+        assert np.array_equal(got[..., col], want[..., col])  # infinities
+        assert np.all(np.abs(got[..., ~col] - want[..., ~col]) <= tol[..., ~col])
