@@ -84,6 +84,13 @@ def load_pmc_traffic() -> dict:
 PMC = {}
 
 
+def route(info: dict) -> str:
+    """Kernel of a product, with the form that it runs in where that is not
+    the kernel's own."""
+    form = "" if info["form"] == "plain" else f" ({info['form']} {'x'.join(map(str, info['tile']))})"
+    return info["kernel"] + form
+
+
 def log(msg: str) -> None:
     print(msg, file=sys.stderr, flush=True)
 
@@ -127,7 +134,7 @@ def headline(ta, ex, steps: int, warmup: int, settle_ms: float):
     return dict(
         settle_ms=settled,
         wall_s=wall, ms_per_step=wall / steps * 1e3, value=flops / (wall / steps) / 1e12,
-        kernel_ms=kernel_ns / 1e6, achieved=flops / kernel_ns / 1e3, kernel=info["kernel"],
+        kernel_ms=kernel_ns / 1e6, achieved=flops / kernel_ns / 1e3, kernel=route(info),
         rel_err=rel, inputs=(ha, hb),
     )
 
@@ -213,7 +220,7 @@ def batched_gelu(ta, ex, iters=10):
     ns = median_ns([ex.run_ops([op]) for _ in range(iters)])
     flops = 2.0 * bt * m * n * k
     return dict(kernel_ms=ns / 1e6, tflops=flops / ns / 1e3, frac=flops / ns / 1e3 / PEAK_F32_SPLIT,
-                kernel=ex.dispatch_info_for(bt, m, n, k)["kernel"],
+                kernel=route(ex.dispatch_info_for(bt, m, n, k)),
                 roofline=roofline("mfma", flops / ns / 1e3, PEAK_F32_SPLIT, "TFLOP/s",
                                   PMC.get("gelu_8x2048")))
 
@@ -304,7 +311,7 @@ def prefill_layer(ta, ex, iters=10):
         # A f32, W f16, C f32 (+ D f32 for the binary epilogues)
         nbytes = 4.0 * mm * kk + 2.0 * kk * nn + 4.0 * mm * nn * (2 if ops[0].epilogue.binary else 1)
         out[name] = dict(us=ns / 1e3, tflops=flops / ns / 1e3,
-                         kernel=ex.dispatch_info_for(1, mm, nn, kk, True)["kernel"],
+                         kernel=route(ex.dispatch_info_for(1, mm, nn, kk, True)),
                          roofline=time_roofline(flops, nbytes, ns * 1e-9, PEAK_FP16_MFMA,
                                                 PMC.get(f"prefill_{name.split('_')[0]}")))
         total_ns += ns

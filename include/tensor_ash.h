@@ -99,12 +99,20 @@ typedef struct ta_copy_desc {
   uint32_t dst_strides[3];
 } ta_copy_desc;
 
-/* ref tensor_ash.h:96-104. */
+/* ta_dispatch_info.form: how the named kernel's product runs. */
+enum {
+  TA_FORM_PLAIN = 0,          /* as named */
+  TA_FORM_SPLIT_PRODUCTS = 1, /* as piece products on the bf16 matrix cores; `tile` is theirs */
+  TA_FORM_K_GROUPS = 2        /* K of a tile shared by four groups of waves */
+};
+
+/* ref tensor_ash.h:96-104; `form` lies in what was tail padding. */
 typedef struct ta_dispatch_info {
   const char *kernel;
   uint32_t tile[3];
   uint32_t has_split_k2;
   uint32_t split_k2_splits;
+  uint32_t form;
 } ta_dispatch_info;
 
 const char *ta_version(void);    /* ref tensor_ash.h:106 */

@@ -934,6 +934,7 @@ int ta_dispatch_info_for(const ta_executor *exec, uint32_t batch, uint32_t m, ui
     out->tile[2] = info.tile[2];
     out->has_split_k2 = info.split_k2_splits ? 1u : 0u;
     out->split_k2_splits = info.split_k2_splits.value_or(0);
+    out->form = (uint32_t)info.form;
   });
 }
 

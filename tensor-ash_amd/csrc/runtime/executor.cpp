@@ -3074,22 +3074,30 @@ DispatchInfo Executor::dispatch_info(uint32_t batch, uint32_t m, uint32_t n, uin
 // src/executor/mod.rs:156-172.
 DispatchInfo Executor::dispatch_info_for(uint32_t batch, uint32_t m, uint32_t n, uint32_t k,
                                          bool b_f16) const {
-  OpPlan p = impl_->plan_shape(batch, m, n, k, b_f16, true);
-  if (!b_f16) {
-    ResolvedMatmul d;
-    d.batch = batch;
-    d.m = m;
-    d.n = n;
-    d.k = k;
-    d.batch_stride_a = d.batch_stride_b = batch > 1 ? 1 : 0;
-    d.total_flops = 2ull * batch * m * n * k;
-    impl_->choose_x6(d, p);
-  }
+  ResolvedMatmul d;
+  d.batch = batch;
+  d.m = m;
+  d.n = n;
+  d.k = k;
+  d.b_f16 = b_f16;
+  d.batch_stride_a = d.batch_stride_b = batch > 1 ? 1 : 0;
+  d.total_flops = 2ull * batch * m * n * k;
+  const OpPlan p = impl_->plan_matmul(d, true);
+  const uint32_t cus = impl_->ctx->cu_count();
   const KernelSpec &s = p.splitk2 ? splitk_stage1_spec(m, n, k) : KERNEL_SPECS[p.kernel];
   DispatchInfo info;
   info.kernel = s.name;
   info.tile = {s.tile_m, s.tile_n, s.tile_k};
   info.split_k2_splits = p.splitk2;
+  if (p.x6) {
+    info.form = DispatchForm::SplitProducts;
+    info.tile = {p.x6, p.x6, 16 * ta_x6_groups(p.x6)};
+  } else if (p.w3) {
+    info.form = DispatchForm::SplitProducts;
+    info.tile = {w3_plan(cus, d).rows, TA_W3_BN, TA_W3_BK};
+  } else if (!p.splitk2 && f32_groups_ok(cus, d, s, 1) && !f32_mi16_ok(d, s.tile_m, s.tile_n, 1)) {
+    info.form = DispatchForm::KGroups;
+  }
   return info;
 }
 

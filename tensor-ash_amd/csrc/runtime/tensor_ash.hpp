@@ -438,10 +438,15 @@ struct RunStats {
 };
 
 // src/executor/mod.rs:64-81.
+// How the named kernel's product runs: as it is, as piece products on the
+// bf16 matrix cores (`tile` is then theirs), or in four K groups.
+enum class DispatchForm : uint32_t { Plain = 0, SplitProducts = 1, KGroups = 2 };
+
 struct DispatchInfo {
   const char *kernel = "";
   std::array<uint32_t, 3> tile{0, 0, 0};
   std::optional<uint32_t> split_k2_splits;
+  DispatchForm form = DispatchForm::Plain;
 };
 
 // src/executor/mod.rs:86-100.

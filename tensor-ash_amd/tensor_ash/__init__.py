@@ -112,7 +112,10 @@ class _ExecOp(C.Structure):
 
 class _DispatchInfo(C.Structure):
     _fields_ = [("kernel", C.c_char_p), ("tile", C.c_uint32 * 3), ("has_split_k2", C.c_uint32),
-                ("split_k2_splits", C.c_uint32)]
+                ("split_k2_splits", C.c_uint32), ("form", C.c_uint32)]
+
+
+_FORMS = ("plain", "split_products", "k_groups")
 
 
 def _sig(name, restype, *argtypes):
@@ -899,7 +902,8 @@ class Executor:
         info = _DispatchInfo()
         _check(_lib.ta_dispatch_info_for(self._h, batch, m, n, k, int(b_f16), C.byref(info)))
         return {"kernel": info.kernel.decode(), "tile": tuple(info.tile),
-                "split_k2": info.split_k2_splits if info.has_split_k2 else None}
+                "split_k2": info.split_k2_splits if info.has_split_k2 else None,
+                "form": _FORMS[info.form]}
 
     def tune_shape(self, batch: int, m: int, n: int, k: int) -> None:
         _check(_lib.ta_tune_shape(self._h, batch, m, n, k))

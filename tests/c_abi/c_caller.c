@@ -72,7 +72,7 @@ static void layout(void) {
   F(ta_copy_desc, extent); F(ta_copy_desc, src_offset); F(ta_copy_desc, src_strides);
   F(ta_copy_desc, dst_offset); F(ta_copy_desc, dst_strides); Z(ta_copy_desc);
   F(ta_dispatch_info, kernel); F(ta_dispatch_info, tile); F(ta_dispatch_info, has_split_k2);
-  F(ta_dispatch_info, split_k2_splits); Z(ta_dispatch_info);
+  F(ta_dispatch_info, split_k2_splits); F(ta_dispatch_info, form); Z(ta_dispatch_info);
   F(ta_matmul_op_v2, base); F(ta_matmul_op_v2, packed_b); F(ta_matmul_op_v2, reserved); Z(ta_matmul_op_v2);
   F(ta_store_desc, head_dim); F(ta_store_desc, pos_base); F(ta_store_desc, pos_scale);
   F(ta_store_desc, stride_head); F(ta_store_desc, stride_dim); F(ta_store_desc, reserved);

@@ -158,3 +158,27 @@ def test_deep_k_route(ta, ex, oracle, monkeypatch, m, n, k, form):
     ta_, tb, c = ex.tensor_from(a), ex.tensor_from(b), ex.tensor([m, n])
     ex.run_ops([ta.MatmulOp(ta_, tb, c)])
     assert np.array_equal(ex.download(c), named)
+
+
+def test_dispatch_info_tells_the_form_that_runs(ta, ex, monkeypatch):
+    """`kernel` stays the registry's name (an explicit selection of it runs the
+    plain form); `form` and `tile` say what an untuned product runs in: the
+    same bits as that form fixed by the environment."""
+    rng = np.random.default_rng(5)
+    m, n, k = 300, 520, 1000
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    monkeypatch.delenv("TA_F32X6", raising=False)
+    info = ex.dispatch_info_for(1, m, n, k)
+    assert info["form"] == "split_products" and info["tile"][0] in TILES and not info["split_k2"]
+    ta_, tb, c = ex.tensor_from(a), ex.tensor_from(b), ex.tensor([m, n])
+    ex.run_ops([ta.MatmulOp(ta_, tb, c)])
+    np.testing.assert_array_equal(ex.download(c), product(ta, ex, a, b, monkeypatch, info["tile"][0]))
+    monkeypatch.setenv("TA_F32X6", "0")
+    plain = ex.dispatch_info_for(1, m, n, k)
+    assert plain["kernel"] == info["kernel"] and plain["form"] != "split_products"
+    assert ex.dispatch_info_for(1, 64, 64, 512)["form"] == "k_groups"
+    w = ex.dispatch_info_for(1, 16, 4096, 14336, True)
+    assert (w["form"], w["tile"]) == ("split_products", (32, 64, 64))
+    assert ex.dispatch_info_for(1, 1, 4096, 4096, True)["form"] == "plain"
+    named = ta.Executor(ex.ctx, kernel_selection=info["kernel"])
+    assert named.dispatch_info_for(1, m, n, k)["form"] != "split_products"
