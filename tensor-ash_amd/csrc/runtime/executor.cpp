@@ -356,15 +356,22 @@ struct ExecutorImpl {
 
   // The heuristic's pick may run in its split-product form; an explicit
   // kernel selection, or a tuned kernel or split count that differs from
-  // the heuristic's, runs as named.
-  void choose_x6(const ResolvedMatmul &d, OpPlan &plan) const {
+  // the heuristic's, runs as named.  The heuristic's kernel alone in the
+  // tuner's store means that nothing beat the untuned route, so the form is
+  // chosen as it is untuned.
+  void choose_x6(const ResolvedMatmul &d, OpPlan &plan, bool splitk_eligible) const {
     if (!selection.is_auto() || KERNEL_SPECS[plan.kernel].kind != KernelKind::GemmF32)
       return;
     const uint32_t cus = ctx->cu_count();
     const size_t heur = heuristic_kernel_index(cus, d.batch, d.m, d.n, d.k, false, false);
-    if (auto e = tuned_entry(TuneKey{d.batch, d.m, d.n, d.k, false}))
+    std::optional<uint32_t> replaces = plan.splitk2;
+    if (auto e = tuned_entry(TuneKey{d.batch, d.m, d.n, d.k, false})) {
       if (e->kernel != heur || e->splitk2_splits)
         return;
+      const auto splits = heuristic_splits(cus, d.batch, d.m, d.n, d.k);
+      if (splitk_eligible && splits && auto_route_fits(d.batch, d.m, d.n, d.k, *splits))
+        replaces = splits;
+    }
     // TA_F32X6 fixes the form (route control): 0, or the tile.
     if (const char *env = std::getenv("TA_F32X6")) {
       const uint32_t tile = (uint32_t)std::strtoul(env, nullptr, 10);
@@ -372,7 +379,8 @@ struct ExecutorImpl {
                       f32x6_plan(d, tile).bytes <= kF32X6ScratchCapBytes;
       plan.x6 = ok ? tile : 0;
     } else {
-      plan.x6 = f32x6_tile(cus, d, KERNEL_SPECS[plan.splitk2 ? plan.kernel : heur], plan.splitk2);
+      plan.x6 = f32x6_tile(cus, d, replaces ? splitk_stage1_spec(d.m, d.n, d.k) : KERNEL_SPECS[heur],
+                           replaces);
     }
     if (plan.x6) {
       plan.splitk2.reset();
@@ -417,7 +425,7 @@ struct ExecutorImpl {
       return p;
     }
     OpPlan p = plan_shape(d.batch, d.m, d.n, d.k, d.b_f16, splitk_eligible);
-    choose_x6(d, p);
+    choose_x6(d, p, splitk_eligible);
     // The heuristic's pick for few rows (as above, not a named or tuned one).
     p.w3 = selection.is_auto() && KERNEL_SPECS[p.kernel].kind == KernelKind::GemmF16w && w3_ok(d) &&
            !std::getenv("TA_NO_W3") &&
@@ -1796,15 +1804,21 @@ struct ExecutorImpl {
   }
 
   std::optional<uint64_t> run_forced_once(const MatmulOp &op, const ResolvedMatmul &d,
-                                          size_t kernel, std::optional<uint32_t> splits) const {
+                                          const OpPlan &p) const {
     ExecutorImpl *self = const_cast<ExecutorImpl *>(this);
     Lease lease(self);
+    return submit_and_wait(lease.s, {op}, {d}, {p});
+  }
+  static OpPlan forced_plan(size_t kernel, std::optional<uint32_t> splits) {
     OpPlan p;
     p.kernel = kernel;
     p.splitk2 = splits;
-    return submit_and_wait(lease.s, {op}, {d}, {p});
+    return p;
   }
 
+  // Measured in turn: every kernel that can run the shape, and the route
+  // that the shape takes untuned where that is another one (split products,
+  // split-K); then split counts.  tune_pick says what is stored.
   void tune_op(const MatmulOp &op, const ResolvedMatmul &d) {
     std::vector<size_t> cands = tune_candidate_indices(d);
     if (cands.empty())
@@ -1813,55 +1827,58 @@ struct ExecutorImpl {
         heuristic_kernel_index(ctx->cu_count(), d.batch, d.m, d.n, d.k, d.b_f16, d.packed_b);
     const double est_ms = (double)d.total_flops / 50e12 * 1e3;
     const uint32_t rounds = est_ms > 8.0 ? 2 : 4;
-    (void)run_forced_once(op, d, std::count(cands.begin(), cands.end(), heur) ? heur : cands[0],
-                          std::nullopt);
-    std::vector<std::vector<uint64_t>> samples(cands.size());
+    std::vector<OpPlan> forms;
+    for (size_t c : cands)
+      forms.push_back(forced_plan(c, std::nullopt));
+    const OpPlan untuned = plan_matmul(d, true);
+    TuneBase base;
+    base.kernel = heur;
+    base.splits = untuned.splitk2;
+    base.split_products = untuned.x6 || untuned.w3;
+    if (base.splits || base.split_products)
+      forms.push_back(untuned);
+    (void)run_forced_once(op, d, forms[std::count(cands.begin(), cands.end(), heur)
+                                           ? std::find(cands.begin(), cands.end(), heur) - cands.begin()
+                                           : 0]);
+    std::vector<std::vector<uint64_t>> samples(forms.size());
     for (uint32_t round = 0; round <= rounds; ++round)
-      for (size_t off = 0; off < cands.size(); ++off) {
-        const size_t ci = candidate_at(cands.size(), round, off);
-        auto ns = run_forced_once(op, d, cands[ci], std::nullopt);
+      for (size_t off = 0; off < forms.size(); ++off) {
+        const size_t ci = candidate_at(forms.size(), round, off);
+        auto ns = run_forced_once(op, d, forms[ci]);
         if (round > 0 && ns)
           samples[ci].push_back(*ns);
       }
-    std::optional<uint64_t> heur_ns;
-    size_t win = cands[0];
-    std::optional<uint64_t> win_ns;
+    std::vector<std::pair<size_t, uint64_t>> kernels;
+    std::vector<std::pair<uint32_t, uint64_t>> split_counts;
     const bool log = std::getenv("TA_LOG") != nullptr;
-    for (size_t i = 0; i < cands.size(); ++i) {
+    for (size_t i = 0; i < forms.size(); ++i) {
       auto md = median(samples[i]);
+      const bool other = i == cands.size(); // the untuned route
       if (log)
         std::fprintf(stderr, "tensor-ash: tune B=%u %ux%ux%u candidate %s: median %.2f us (%zu samples)%s\n",
-                     d.batch, d.m, d.n, d.k, KERNEL_SPECS[cands[i]].name,
+                     d.batch, d.m, d.n, d.k, KERNEL_SPECS[forms[i].kernel].name,
                      md ? (double)*md / 1e3 : -1.0, samples[i].size(),
-                     cands[i] == heur ? " [heuristic]" : "");
+                     other                      ? " [untuned route]"
+                     : forms[i].kernel == heur ? " [heuristic]"
+                                                : "");
       if (!md)
         continue;
-      if (cands[i] == heur)
-        heur_ns = md;
-      if (!win_ns || *md < *win_ns) {
-        win_ns = md;
-        win = cands[i];
-      }
-    }
-    if (!win_ns)
-      fail("no candidate produced a measurement");
-    if (heur_ns && (double)*win_ns >= (double)*heur_ns * 0.98) {
-      win = heur;
-      win_ns = heur_ns;
+      if (other || (forms.size() == cands.size() && cands[i] == heur))
+        base.ns = md;
+      if (!other)
+        kernels.push_back({cands[i], *md});
     }
     // Reduction pass: probe split-K against the DP winner on deep-K,
     // few-tile shapes (executor/tuning.rs:203-250).
-    std::optional<uint32_t> best_splits;
     const KernelSpec &s1 = splitk_stage1_spec(d.m, d.n, d.k);
     const uint64_t tiles = (uint64_t)d.batch * div_ceil(d.m, s1.tile_m) * div_ceil(d.n, s1.tile_n);
     if (!d.b_f16 && !d.packed_b && d.k >= 1024 && tiles < ctx->cu_count()) {
-      std::optional<uint64_t> best;
       for (uint32_t splits : {4u, 8u, 16u, 32u, 64u, 128u}) {
         if (d.k / splits < 128 || !auto_route_fits(d.batch, d.m, d.n, d.k, splits))
           continue;
         std::vector<uint64_t> ss;
         for (uint32_t r = 0; r <= rounds; ++r) {
-          auto ns = run_forced_once(op, d, registry_index(s1.name), splits);
+          auto ns = run_forced_once(op, d, forced_plan(registry_index(s1.name), splits));
           if (r > 0 && ns)
             ss.push_back(*ns);
         }
@@ -1869,19 +1886,20 @@ struct ExecutorImpl {
         if (log)
           std::fprintf(stderr, "tensor-ash: tune B=%u %ux%ux%u split-K %s x %u: median %.2f us\n",
                        d.batch, d.m, d.n, d.k, s1.name, splits, md ? (double)*md / 1e3 : -1.0);
-        if (md && (!best || *md < *best)) {
-          best = md;
-          best_splits = splits;
-        }
+        if (md)
+          split_counts.push_back({splits, *md});
       }
-      if (!best || (double)*best >= (double)*win_ns * 0.98)
-        best_splits.reset();
     }
-    record_tuned(TuneKey{d.batch, d.m, d.n, d.k, d.b_f16}, TuneEntry{win, best_splits});
+    const auto pick = tune_pick(base, kernels, split_counts);
+    if (!pick)
+      fail("no candidate produced a measurement");
+    record_tuned(TuneKey{d.batch, d.m, d.n, d.k, d.b_f16}, *pick);
     if (std::getenv("TA_LOG"))
       std::fprintf(stderr, "tensor-ash: tuned B=%u %ux%ux%u: %s%s\n", d.batch, d.m, d.n, d.k,
-                   KERNEL_SPECS[win].name,
-                   best_splits ? (" + splitk2=" + std::to_string(*best_splits)).c_str() : "");
+                   KERNEL_SPECS[pick->kernel].name,
+                   pick->splitk2_splits
+                       ? (" + splitk2=" + std::to_string(*pick->splitk2_splits)).c_str()
+                       : "");
   }
 
   // ---- run_ops (src/executor/dispatch.rs:87-188) ----
@@ -2013,10 +2031,10 @@ struct ExecutorImpl {
   }
 
   // The route of an explicit split count: the split-K stage-1 tile plus
-  // the reduce for splits > 1, else the data-parallel route (the same
-  // plan run_ops gives an op that may not split), which needs no scratch
-  // for f32 operands.  The allocating and the allocation-free entry
-  // points share it, so they launch the same kernels.
+  // the reduce for splits > 1, else the data-parallel route on the FP32
+  // MFMAs, which needs no scratch for f32 operands (run_ops may run the op
+  // as split products).  The allocating and the allocation-free entry points
+  // share it, so they launch the same kernels.
   OpPlan split_k2_plan(const MatmulOp &op, const ResolvedMatmul &d, uint32_t splits) const {
     if (splits <= 1) {
       // on the FP32 MFMAs: the allocation-free form has no room for packed

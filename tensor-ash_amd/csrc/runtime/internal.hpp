@@ -226,6 +226,19 @@ struct TuneEntry {
   size_t kernel;
   std::optional<uint32_t> splitk2_splits;
 };
+// The route a shape takes untuned, as measured: `kernel` as it is, its
+// split-product form, or split-K.
+struct TuneBase {
+  size_t kernel = 0;
+  std::optional<uint32_t> splits;
+  bool split_products = false;
+  std::optional<uint64_t> ns;
+};
+// What the tuner stores: the untuned route unless a kernel, or a split
+// count, is more than 2% faster.  Nothing measured: nothing.
+std::optional<TuneEntry> tune_pick(const TuneBase &base,
+                                   const std::vector<std::pair<size_t, uint64_t>> &kernels,
+                                   const std::vector<std::pair<uint32_t, uint64_t>> &split_counts);
 std::string tune_store_path(const Context &ctx);
 std::string tune_header_line(const Context &ctx);
 std::map<TuneKey, TuneEntry> parse_tune_store(const std::string &text, const std::string &header);

@@ -658,6 +658,37 @@ bool TuneKey::operator<(const TuneKey &o) const {
   return std::tie(batch, m, n, k, b_f16) < std::tie(o.batch, o.m, o.n, o.k, o.b_f16);
 }
 
+std::optional<TuneEntry> tune_pick(const TuneBase &base,
+                                   const std::vector<std::pair<size_t, uint64_t>> &kernels,
+                                   const std::vector<std::pair<uint32_t, uint64_t>> &split_counts) {
+  std::optional<TuneEntry> pick;
+  uint64_t pick_ns = 0;
+  auto offer = [&](const TuneEntry &e, uint64_t ns) {
+    if (!pick || (double)ns < (double)pick_ns * 0.98) {
+      pick = e;
+      pick_ns = ns;
+    }
+  };
+  if (base.ns)
+    offer(TuneEntry{base.kernel, base.splits}, *base.ns);
+  auto fastest = [](const auto &list, auto skip) {
+    auto best = list.end();
+    for (auto it = list.begin(); it != list.end(); ++it)
+      if (!skip(it->first) && (best == list.end() || it->second < best->second))
+        best = it;
+    return best;
+  };
+  // The heuristic's kernel by itself stands for its split-product form where
+  // the untuned route is that one, so its plain form cannot be stored.
+  const auto k = fastest(kernels, [&](size_t i) { return base.split_products && i == base.kernel; });
+  if (k != kernels.end())
+    offer(TuneEntry{k->first, std::nullopt}, k->second);
+  const auto s = fastest(split_counts, [](uint32_t) { return false; });
+  if (s != split_counts.end())
+    offer(TuneEntry{pick ? pick->kernel : base.kernel, s->first}, s->second);
+  return pick;
+}
+
 // Persistent store (src/pipeline/tuning.rs:60-199): one header line that
 // binds the HIP runtime version, the gfx arch and a hash of every loaded
 // code object, then "B M N K kernel [splitk2=S] [bf16]" lines.

@@ -264,6 +264,33 @@ static void test_tuner_helpers() {
     for (size_t v : rank_sums)
       CHECK(v == rank_sums[0]);
   }
+  // what is stored: the untuned route, whatever its form, unless something
+  // else is more than 2% faster
+  {
+    const size_t heur = registry_index("f32_m64n64"), other = registry_index("f32_m128n64");
+    auto picked = [&](bool pieces, std::optional<uint32_t> base_splits, std::optional<uint64_t> base_ns,
+                      uint64_t heur_ns, uint64_t other_ns, std::vector<std::pair<uint32_t, uint64_t>> sk,
+                      size_t kernel, std::optional<uint32_t> splits) {
+      TuneBase b;
+      b.kernel = heur;
+      b.splits = base_splits;
+      b.split_products = pieces;
+      b.ns = base_ns;
+      const auto e = tune_pick(b, {{heur, heur_ns}, {other, other_ns}}, sk);
+      return e && e->kernel == kernel && e->splitk2_splits == splits;
+    };
+    const auto none = std::optional<uint32_t>{};
+    CHECK(picked(false, none, 1000, 1000, 985, {}, heur, none));
+    CHECK(picked(false, none, 1000, 1000, 970, {}, other, none));
+    CHECK(picked(false, none, 1000, 1000, 970, {{4, 960}, {8, 900}}, other, 8u));
+    CHECK(picked(true, none, 300, 736, 700, {{4, 500}}, heur, none)); // split products stay
+    CHECK(picked(true, none, 300, 200, 250, {}, other, none)); // `heur` alone would mean the pieces
+    CHECK(picked(true, none, 300, 736, 700, {{8, 200}}, heur, 8u));
+    CHECK(picked(false, 12u, 300, 900, 700, {{8, 299}}, heur, 12u)); // so does untuned split-K
+    CHECK(picked(false, 12u, 300, 900, 250, {{8, 260}}, other, none));
+    CHECK(picked(true, none, {}, 736, 700, {}, other, none)); // the pieces were not measured
+    CHECK(!tune_pick(TuneBase{}, {}, {}));
+  }
   // tune store: round trip, header binding, malformed lines skipped
   std::map<TuneKey, TuneEntry> m;
   m[TuneKey{1, 64, 256, 65536, false}] = TuneEntry{registry_index("f32_m64n64"), 32u};

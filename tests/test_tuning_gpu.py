@@ -78,3 +78,25 @@ def test_stale_store_is_ignored(ta, ctx, cache_dir):
         (d / name).write_text("tensor-ash-tune-v3 stale header\n1 4096 4096 4096 f32_m64n64\n")
     ex = ta.Executor(ctx, tune=False)
     assert ex.dispatch_info_for(1, 4096, 4096, 4096)["kernel"] == "f32_m256n256"
+
+
+@pytest.mark.parametrize("m,n,k,f16", [(1536, 360, 1336, False), (16, 4096, 14336, True)])
+def test_tuning_measures_the_untuned_route(ta, ctx, cache_dir, m, n, k, f16):
+    """The split-product form of a product is a candidate of its own: the FP32
+    MFMA kernels, at less than half its speed here, do not switch it off (an
+    f16-MFMA kernel, which rounds A, may)."""
+    ex = ta.Executor(ctx, tune=True)
+    rng = np.random.default_rng(3)
+    a = ex.tensor_from(rng.standard_normal((m, k)).astype(np.float32))
+    b = ex.tensor_from(rng.standard_normal((k, n)).astype(np.float32), f16=f16)
+    c = ex.tensor([m, n])
+    before = ex.dispatch_info_for(1, m, n, k, f16)
+    assert before["form"] == "split_products"
+    ex.run_ops([ta.MatmulOp(a, b, c)])
+    lines = store_lines(cache_dir)
+    winner = lines[0].split()[4]
+    fresh = ta.Executor(ctx, tune=False)
+    for e in (ex, fresh):
+        after = e.dispatch_info_for(1, m, n, k, f16)
+        assert after["kernel"] == winner
+        assert after == before or winner.startswith(("f16w_mfma", "f16w_sk")), after
