@@ -79,54 +79,110 @@ TA_DEVICE float half_max(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-// One wave's 32 query rows in plain f32 arithmetic, for rows whose result
-// is not finite: an infinite operand must not meet the zero pieces of a
-// split one (inf * 0), so these rows are computed again with whole values.
+// One wave's 32 query rows on the f32 MFMAs, for rows whose result is not
+// finite: an infinite operand must not meet the zero pieces of a split one
+// (inf * 0), so these rows are computed again with whole values, from the
+// caches as they lie in memory.  Blocks of 32 keys that some row does not
+// attend to in full add their values row by row: a masked probability is a
+// zero too.  With an infinite value in every head: 2048 tokens, 32 heads / 8
+// KV, dh 128, f16 863 us; 512 tokens at 512, 32 / 8, dh 64, f32 q 211 us (a
+// lane per key and column: 15300 and 5200).  Two loops, not a branch in one:
+// the joined registers cost the split form a wave per SIMD.
 template <int DH, bool IO16>
-TA_DEVICE void flash_rows_plain(const FlashArgs &p, uint32_t head, uint32_t kv_head, uint32_t row0,
+TA_DEVICE void flash_rows_whole(const FlashArgs &p, uint32_t head, uint32_t kv_head, uint32_t row0,
                                 uint32_t lane) {
+  constexpr int HALF = DH / 2, DB = DH / 32;
+  const uint32_t j = lane & 31u, h = lane >> 5, row = row0 + j;
+  const bool live = row < p.t_q;
   const _Float16 *kt = static_cast<const _Float16 *>(p.kt) + (uint64_t)kv_head * DH * p.t_max;
   const _Float16 *vv = static_cast<const _Float16 *>(p.v) + (uint64_t)kv_head * p.t_max * DH;
+  const uint32_t keys = min(p.kv_len, p.t_max);
+  const uint32_t valid = live ? min(keys, p.pos_base + row + 1u) : 0u;
+  const uint32_t any = min(keys, p.pos_base + min(row0 + 32u, p.t_q));
+  const uint32_t all = min(keys, p.pos_base + row0 + 1u);
+  const uint64_t qbase = (uint64_t)head * p.q_head_stride + (uint64_t)min(row, p.t_q - 1u) * p.q_row_stride;
   const float scale2 = p.scale * 1.44269504088896340736f;
-  for (uint32_t row = row0; row < min(row0 + 32u, p.t_q); ++row) {
-    const uint32_t valid = min(min(p.kv_len, p.pos_base + row + 1u), p.t_max);
-    const uint64_t qbase = (uint64_t)head * p.q_head_stride + (uint64_t)row * p.q_row_stride;
-    auto score = [&](uint32_t key) {
-      float acc = 0.0f;
-      for (uint32_t d = 0; d < (uint32_t)DH; ++d)
-        acc = fmaf(IO16 ? (float)static_cast<const _Float16 *>(p.q)[qbase + d]
-                        : static_cast<const float *>(p.q)[qbase + d],
-                   (float)kt[(uint64_t)d * p.t_max + key], acc);
-      return acc * scale2;
-    };
-    float m = kNegMax;
-    for (uint32_t key = lane; key < valid; key += 64u)
-      m = fmaxf(m, score(key));
-    for (int x = 32; x > 0; x >>= 1)
-      m = fmaxf(m, __shfl_xor(m, x));
-    float l = 0.0f, acc[DH / 64];
-    for (int i = 0; i < DH / 64; ++i)
-      acc[i] = 0.0f;
-    for (uint32_t k0 = 0; k0 < valid; k0 += 64u) {
-      const float pk = k0 + lane < valid ? exp2f(score(k0 + lane) - m) : 0.0f;
-      l += pk;
-      for (uint32_t k = 0; k < min(64u, valid - k0); ++k) {
-        const float w = __shfl(pk, (int)k);
-        for (int i = 0; i < DH / 64; ++i)
-          acc[i] = fmaf(w, (float)vv[(uint64_t)(k0 + k) * DH + i * 64 + lane], acc[i]);
+  f32x16 o[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+    o[b] = f32x16{};
+  float m_run = kNegMax, l_run = 0.0f;
+  f32x16 s;
+  // Register e of s: the probability of key k0 + 4 h + 8 (e / 4) + e % 4.
+  auto block = [&](uint32_t k0) __attribute__((always_inline)) {
+    s = f32x16{};
+    const uint32_t key = min(k0 + j, any - 1u); // keys past the rows' are masked
+#pragma unroll 4
+    for (uint32_t d = h * HALF; d < (h + 1u) * HALF; ++d) {
+      const float q = IO16 ? (float)static_cast<const _Float16 *>(p.q)[qbase + d]
+                           : static_cast<const float *>(p.q)[qbase + d];
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32((float)kt[(uint64_t)d * p.t_max + key], q, s, 0, 0, 0);
+    }
+    const uint32_t kbase = k0 + 4u * h;
+    float m_new = m_run;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = kbase + 8u * (e / 4) + e % 4 < valid ? s[e] * scale2 : kNegMax;
+      m_new = fmaxf(m_new, s[e]);
+    }
+    m_new = fmaxf(m_new, __shfl_xor(m_new, 32));
+    const float corr = exp2f(m_run - m_new);
+    m_run = m_new;
+    float psum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = kbase + 8u * (e / 4) + e % 4 < valid ? exp2f(s[e] - m_new) : 0.0f;
+      psum += s[e];
+    }
+    l_run = l_run * corr + psum;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        o[b][e] *= corr;
+  };
+  uint32_t k0 = 0;
+  for (; k0 + 32u <= all; k0 += 32u) {
+    block(k0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+        o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            (float)vv[(uint64_t)(k0 + 4u * h + 8u * (e / 4) + e % 4) * DH + b * 32 + j], s[e], o[b], 0, 0, 0);
+  }
+  for (; k0 < any; k0 += 32u) {
+    block(k0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float other = __shfl_xor(s[e], 32);
+#pragma unroll
+      for (uint32_t half = 0; half < 2u; ++half) {
+        const uint32_t at = k0 + 4u * half + 8u * (e / 4) + e % 4;
+        const float w = half == h ? s[e] : other;
+        const _Float16 *v = vv + (uint64_t)min(at, any - 1u) * DH + 4u * h;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f16x4 x = *reinterpret_cast<const f16x4 *>(v + b * 32 + 8 * q);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              o[b][4 * q + r] = at < valid ? fmaf(w, (float)x[r], o[b][4 * q + r]) : o[b][4 * q + r];
+          }
       }
     }
-    for (int x = 32; x > 0; x >>= 1)
-      l += __shfl_xor(l, x);
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const uint64_t obase = (uint64_t)head * p.o_head_stride + (uint64_t)row * p.o_row_stride;
-    for (int i = 0; i < DH / 64; ++i) {
-      const uint64_t at = obase + i * 64 + lane;
-      if constexpr (IO16)
-        static_cast<_Float16 *>(p.out)[at] = (_Float16)(acc[i] * inv);
-      else
-        static_cast<float *>(p.out)[at] = acc[i] * inv;
-    }
+  }
+  const float l = l_run + __shfl_xor(l_run, 32);
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  if (live) {
+    const uint64_t obase = (uint64_t)head * p.o_head_stride + (uint64_t)row * p.o_row_stride + 4u * h;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        store4<IO16>(p.out, obase + b * 32 + 8 * q,
+                     f32x4{o[b][4 * q] * inv, o[b][4 * q + 1] * inv, o[b][4 * q + 2] * inv, o[b][4 * q + 3] * inv});
   }
 }
 
@@ -358,7 +414,7 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 //    to 2^-18, and 2^-36 absolute below that); the row sum takes the f32 p.
 // Measured against f64 (normal inputs): 1.7e-7 .. 3.5e-7, as the f32 MFMA
 // kernel had.  An infinite operand would meet zero pieces (inf * 0); rows
-// that come out non-finite are computed again by flash_rows_plain.
+// that come out non-finite are computed again by flash_rows_whole.
 //
 // Layout.  K and V tiles stay in LDS as they lie in the caches ([d][key],
 // [key][d]), and both reach the matrix cores through ds_read_b64_tr_b16.
@@ -773,7 +829,7 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
                        f32x4{o[b][4 * q], o[b][4 * q + 1], o[b][4 * q + 2], o[b][4 * q + 3]});
     }
     if (__any(live && !finite))
-      flash_rows_plain<DH, IO16>(p, head, kv_head, qw0, lane);
+      flash_rows_whole<DH, IO16>(p, head, kv_head, qw0, lane);
   }
 };
 

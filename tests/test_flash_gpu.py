@@ -299,3 +299,29 @@ def test_flash_f16_cache_infinities(ta, ex, oracle, dh, t_q, io16):
     hit[0, 40:, 5] = True
     assert np.all(np.isposinf(got[hit]))
     assert np.max(np.abs(got[~hit] - ref[~hit])) <= 2e-5 + (2.0 ** -11 if io16 else 0.0)
+
+
+@pytest.mark.parametrize("io16", [False, True], ids=["kv16", "io16"])
+@pytest.mark.parametrize("heads,kv_heads,t_q,t_max,dh,kv_len,pos_base", [
+    (4, 2, 130, 301, 64, 207, 77), (3, 3, 97, 128, 128, 97, 0), (2, 1, 31, 520, 128, 400, 480), (4, 1, 64, 96, 64, 96, 32)])
+def test_flash_f16_cache_rows_computed_whole(ta, ex, oracle, heads, kv_heads, t_q, t_max, dh, kv_len, pos_base, io16):
+    """A key of -inf against positive q in every head: split pieces give NaN
+    for every row that attends to it, so all rows are computed in whole
+    values: full blocks of keys, blocks that cross the causal frontier, and
+    rows past the last one."""
+    q = oracle.round_via_f16(oracle.fill_det(heads * t_q * dh, 5810)).reshape(heads, t_q, dh)
+    q[:, :, 3] = np.abs(q[:, :, 3]) + np.float32(0.25)
+    kt, v = fill_kv(oracle, kv_heads, dh, t_max, kv_len, poison=False)
+    kt, v = oracle.round_via_f16(kt).reshape(kt.shape), oracle.round_via_f16(v).reshape(v.shape)
+    kt[:, 3, 0] = -np.inf
+    kt[:, :, kv_len:], v[:, kv_len:, :] = np.inf, np.inf
+    first = 0 if pos_base else 1  # row 0 at position 0 attends to that key alone
+    out = ex.tensor([heads, t_q, dh], f16=io16)
+    ex.flash_attention(ex.tensor_from(q, f16=io16), ex.tensor_from(kt, f16=True), ex.tensor_from(v, f16=True), out,
+                       ta.FlashAttentionDesc(kv_len, pos_base, 0.125))
+    got = ex.download(out).reshape(heads, t_q, dh)
+    safe_kt, safe_v = kt.copy(), v.copy()
+    safe_kt[:, :, kv_len:], safe_v[:, kv_len:, :] = 0, 0
+    ref = oracle.flash_attention(q, safe_kt, safe_v, heads, kv_heads, t_q, t_max, dh, kv_len, pos_base,
+                                 0.125).reshape(got.shape)
+    assert np.max(np.abs(got[:, first:] - ref[:, first:])) <= 2e-5 + (2.0 ** -11 if io16 else 0.0)
