@@ -42,9 +42,13 @@ template <int DH> constexpr int flash_qblocks() { return ta_flash_qblocks(DH); }
 constexpr float kNegMax = -3.402823466e38f;
 constexpr float kMasked = -__builtin_inff();
 constexpr float kMinScale = 1.17549435e-38f; // 2^-126
-// f16-cache kernels: a row's probabilities stay below 2^kSlack, and are
-// scaled by kProbScale so that their f16 pieces reach down to 2^-35 of it.
-constexpr float kSlack = 4.0f, kProbScale = 2048.0f;
+// f16-cache kernels: a row's reference point (m_run) lies kProbBits below a
+// maximum of its scores, so that its probabilities, at most 2^(kProbBits +
+// kSlack), use the range of their f16 pieces.
+constexpr float kProbBits = 11.0f, kSlack = 4.0f;
+// What the first piece of an f32 operand leaves over is scaled by kLowScale
+// before it becomes f16, and its products are summed apart.
+constexpr float kLowScale = 2048.0f;
 
 template <bool F16> TA_DEVICE void store4(void *base, uint64_t i, f32x4 v) {
   if constexpr (F16) {
@@ -60,8 +64,10 @@ template <bool F16> TA_DEVICE void store4(void *base, uint64_t i, f32x4 v) {
 // XCD (its L2 keeps that head's K/V).  Tiles start longest first over all
 // heads of an XCD: the last tile of a causal prompt has q_tiles times the
 // first one's keys, and head by head the second half of the heads started
-// its longest tiles when the first had drained (2048 tokens, 32 heads, dh
-// 128: SQ_BUSY_CU_CYCLES two thirds of the launch).
+// its longest tiles when the first had drained.  That counts for more than an
+// XCD's own heads where 8 does not divide them (us, head by head in one run
+// per XCD / longest first; 2048 tokens, dh 128: 12 heads f32 215 / 192, f16
+// 52.7 / 45.7; 4 heads 186.5 / 186.9, 30.9 / 31.4).
 TA_DEVICE void flash_work(const FlashArgs &p, uint32_t &head, uint32_t &tile) {
   uint32_t i = blockIdx.x, first = 0, count = p.heads;
   if (p.heads % 8u == 0u) {
@@ -113,7 +119,8 @@ TA_DEVICE void flash_rows_whole(const FlashArgs &p, uint32_t head, uint32_t kv_h
     s = f32x16{};
     const uint32_t key = min(k0 + j, any - 1u); // keys past the rows' are masked
 #pragma unroll 4
-    for (uint32_t d = h * HALF; d < (h + 1u) * HALF; ++d) {
+    for (uint32_t i = 0; i < (uint32_t)HALF; ++i) {
+      const uint32_t d = h * HALF + i;
       const float q = IO16 ? (float)static_cast<const _Float16 *>(p.q)[qbase + d]
                            : static_cast<const float *>(p.q)[qbase + d];
       s = __builtin_amdgcn_mfma_f32_32x32x2f32((float)kt[(uint64_t)d * p.t_max + key], q, s, 0, 0, 0);
@@ -405,13 +412,19 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 
 // ---------------------------------------------------------------------
 // f16 caches: both products on v_mfma_f32_32x32x16_f16 (16 times the f32
-// rate), with f32 accuracy kept by splitting the f32 operands into f16
-// pieces whose products with the f16 cache values are exact in the f32
-// accumulator:
+// rate), with the f32 operands split into f16 pieces whose products with the
+// f16 cache values are exact in the f32 accumulator:
 //  * q: as it is when f16; f32 rows are scaled by a power of two (largest
-//    value into [2^14, 2^15)) and split exactly into three pieces;
-//  * probabilities p: two pieces of p * kProbScale (22 bits of every p down
-//    to 2^-18, and 2^-36 absolute below that); the row sum takes the f32 p.
+//    value into [2^14, 2^15)) and split into three pieces: exactly down to
+//    2^-26 of the row's largest value, to 2^-50 of it below that;
+//  * probabilities: two pieces, within 2^-24 of every value down to 2^-23 of
+//    the row's largest, and to 2^-47 of that below; the row sum takes the f32
+//    values.
+// The pieces after the first are scaled by kLowScale and summed apart: in one
+// sum they end at f16's smallest step, 2^-36 of a row's largest probability
+// and 2^-40 of its largest q, and results that come from keys of 2^-26 alone
+// were 8e-4 off (now 6e-7).  It costs 16 FMAs a tile and 32 columns: 76.6 ->
+// 80.5 us at the first size below, 31.8 -> 35.8 for 16 heads of dh 64.
 // Measured against f64 (normal inputs): 1.7e-7 .. 3.5e-7, as the f32 MFMA
 // kernel had.  An infinite operand would meet zero pieces (inf * 0); rows
 // that come out non-finite are computed again by flash_rows_whole.
@@ -431,10 +444,11 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 // wave; ta_flash16_rows).  Tiles of 128 rows x 64 keys were slower (102
 // against 94 us): fewer, longer workgroups leave CUs idle at the end.
 //
-// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 73 us
-// here (470 TFLOP/s), kv16 434 -> 98 us; 512 tokens, 4 KV heads, dh 64, f16:
-// 28 -> 10.8 us.  MFMAs are busy 33% and the VALU (exp2, splits) about as
-// long; a wave's two phases overlap only with its SIMD's other wave.
+// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 80.5
+// us here (427 TFLOP/s), kv16 434 -> 112 us; 512 tokens, 4 KV heads, dh 64,
+// f16: 28 -> 10.9 us.  MFMAs are busy 30% (kv16 38%) and CUs 75%; a wave's
+// scores, softmax and PV product follow each other and overlap only with its
+// SIMD's other wave.
 template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH16 {
   static constexpr int T = 64 * QB * KP;
   static constexpr int BQ = 32 * QB;         // query rows per workgroup
@@ -536,7 +550,7 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
 #pragma unroll
             for (int q = 0; q < QP; ++q) {
               qf[q][s][i] = (_Float16)x;
-              x -= (float)qf[q][s][i];
+              x = (x - (float)qf[q][s][i]) * (q == 0 ? kLowScale : 1.0f);
             }
           }
       }
@@ -677,10 +691,10 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
       }
       const uint32_t st = lds0 + (t & 1u) * STAGE;
 
-      f32x16 s[KB];
+      f32x16 s[KB], low[KB]; // low: the smaller pieces of q
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
-        s[kb] = f32x16{};
+        s[kb] = low[kb] = f32x16{};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -688,9 +702,18 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
           const uint32_t at = st + k_off[kb] + ks * 16 * (BK * 2);
           const f16x8 a = tr(at, at + 4 * (BK * 2));
 #pragma unroll
-          for (int q = 0; q < QP; ++q)
-            s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[q][ks], s[kb], 0, 0, 0);
+          for (int q = 0; q < QP; ++q) {
+            f32x16 &c = q ? low[kb] : s[kb];
+            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[q][ks], c, 0, 0, 0);
+          }
         }
+      if constexpr (QP > 1) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            s[kb][e] = fmaf(low[kb][e], 1.0f / kLowScale, s[kb][e]);
+      }
 
       float tmax = kNegMax;
       if (kw0 + BKW > wave_all) {
@@ -713,8 +736,8 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
       // by 2^kSlack (probabilities stay below 2^kSlack): with 32 rows in a
       // wave some row finds a new maximum in nearly every tile, and scaling
       // the output for it was a third of the softmax's instructions.
-      if (__any(tmax > m_run + kSlack)) {
-        const float m_new = fmaxf(m_run, tmax);
+      if (__any(tmax > m_run + (kProbBits + kSlack))) {
+        const float m_new = fmaxf(m_run, tmax - kProbBits);
         const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
         l_run *= corr;
@@ -731,45 +754,47 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
         for (int e = 0; e < 16; ++e) {
           const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][e], scale2, -m_run));
           psum += pv;
-          s[kb][e] = pv * kProbScale;
+          s[kb][e] = pv;
         }
       l_run += psum;
 
       // O^T += V^T P^T: step u of a 32-key block pairs P registers 8u..8u+7
       // (keys 16u + 4h + 0..3 and 16u + 8 + 4h + 0..3) with the same V rows.
+      f16x8 hi[KB][2], lo[KB][2];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f16x8 hi, lo;
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int e = 0; e < 8; e += 2) {
             typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
             const float x = s[kb][8 * u + e], y = s[kb][8 * u + e + 1];
             f16x2 a = {(_Float16)x, (_Float16)y};
             asm("" : "+v"(a)); // widen from the packed pair
-            hi[e] = a[0];
-            hi[e + 1] = a[1];
-            lo[e] = (_Float16)(x - (float)a[0]);
-            lo[e + 1] = (_Float16)(y - (float)a[1]);
+            hi[kb][u][e] = a[0];
+            hi[kb][u][e + 1] = a[1];
+            lo[kb][u][e] = (_Float16)fmaf((float)a[0], -kLowScale, x * kLowScale);
+            lo[kb][u][e + 1] = (_Float16)fmaf((float)a[1], -kLowScale, y * kLowScale);
           }
 #pragma unroll
-          for (int b = 0; b < DB; ++b) {
+      for (int b = 0; b < DB; ++b) {
+        f32x16 low = f32x16{};
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
             const uint32_t at = st + v_off[b] + (kb * 32 + u * 16) * (DH * 2);
             const f16x8 a = tr(at, at + 8 * (DH * 2));
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi, o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo, o[b], 0, 0, 0);
+            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi[kb][u], o[b], 0, 0, 0);
+            low = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo[kb][u], low, 0, 0, 0);
           }
-        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          o[b][e] = fmaf(low[e], 1.0f / kLowScale, o[b][e]);
+      }
       if (t + 1 < n_tiles)
         commit(t + 1);
     }
-#pragma unroll
-    for (int b = 0; b < DB; ++b)
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        o[b][e] *= 1.0f / kProbScale;
-
     float m = m_run, l = l_run, a0 = 1.0f;
     float mp[KP], a[KP];
     float *mb = reinterpret_cast<float *>(smem) + qb * ((KP - 1) * REGS * 64);

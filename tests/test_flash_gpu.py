@@ -325,3 +325,53 @@ def test_flash_f16_cache_rows_computed_whole(ta, ex, oracle, heads, kv_heads, t_
     ref = oracle.flash_attention(q, safe_kt, safe_v, heads, kv_heads, t_q, t_max, dh, kv_len, pos_base,
                                  0.125).reshape(got.shape)
     assert np.max(np.abs(got[:, first:] - ref[:, first:])) <= 2e-5 + (2.0 ** -11 if io16 else 0.0)
+
+
+@pytest.mark.parametrize("io16", [False, True], ids=["kv16", "io16"])
+@pytest.mark.parametrize("dh", [64, 128])
+def test_flash_f16_cache_light_keys(ta, ex, dh, io16):
+    """Results that come from keys of small weight alone: key 0 holds nearly
+    all of it and its V is 0.  Weights near 2^-26 come out as f32 arithmetic
+    gives them where results are f32: 2^-24 of a score of 26 in the exponent
+    and as much in a few roundings, below 2^-17 (probabilities kept to 2^-36
+    of the largest: 2^-11).  f16 results keep 2^-24, their own smallest step."""
+    heads, t = 2, 96
+    rng = np.random.default_rng(9)
+    q = np.ones((heads, t, dh), np.float32)
+    kt = np.zeros((heads, dh, t), np.float32)
+    kt[:, 0, 1:] = -(25.0 + rng.uniform(0, 2, (heads, t - 1))).astype(np.float16).astype(np.float32)
+    v = rng.uniform(0.5, 1.5, (heads, t, dh)).astype(np.float16).astype(np.float32)
+    v[:, 0, :] = 0
+    scale = float(np.float32(np.log(2.0)))
+    out = ex.tensor([heads, t, dh], f16=io16)
+    ex.flash_attention(ex.tensor_from(q, f16=io16), ex.tensor_from(kt, f16=True), ex.tensor_from(v, f16=True), out,
+                       ta.FlashAttentionDesc(t, 0, scale))
+    got = ex.download(out).reshape(heads, t, dh).astype(np.float64)
+    s = np.einsum("hqd,hdk->hqk", q.astype(np.float64), kt.astype(np.float64)) * scale
+    p = np.where(np.tril(np.ones((t, t), bool)), np.exp(s), 0.0)
+    ref = (p / p.sum(-1, keepdims=True)) @ v
+    err = np.abs(got[:, 1:] - ref[:, 1:])
+    rel = np.max(err / ref[:, 1:])
+    print(f"relative error {rel:.2e}", flush=True)
+    assert np.max(err) <= 2.0 ** -24 if io16 else rel <= 2.0 ** -17
+
+
+@pytest.mark.parametrize("dh", [64, 128])
+def test_flash_f16_cache_q_over_a_wide_range(ta, ex, oracle, dh):
+    """f32 q whose largest value meets zeros of K: scores come from values
+    2^-27 of it, and stay exact products (2^-40 of the largest alone would
+    leave 13 bits of each)."""
+    heads, t = 2, 70
+    q = oracle.fill_det(heads * t * dh, 5820).reshape(heads, t, dh) * np.float32(2.0 ** -27)
+    q[:, :, 5] = 1.0
+    kt, v = fill_kv(oracle, heads, dh, t, t)
+    kt, v = oracle.round_via_f16(kt).reshape(kt.shape), oracle.round_via_f16(v).reshape(v.shape)
+    kt[:, 5, :] = 0
+    scale = 2.0 ** 27
+    out = ex.tensor([heads, t, dh])
+    ex.flash_attention(ex.tensor_from(q), ex.tensor_from(kt, f16=True), ex.tensor_from(v, f16=True), out,
+                       ta.FlashAttentionDesc(t, 0, scale))
+    ref = oracle.flash_attention(q, kt, v, heads, heads, t, t, dh, t, 0, scale)
+    err, idx = oracle.max_abs_err(ex.download(out).reshape(-1), ref)
+    print(f"error {err:.2e}", flush=True)
+    assert err <= 2e-5, f"err {err} at {idx}"
