@@ -142,6 +142,21 @@ def test_f16w3_small_values_beside_large_ones(ta, ex, small):
     assert np.array_equal(ex.download(c), want.astype(np.float32))
 
 
+@pytest.mark.parametrize("ea,eb", [(-105, -14), (-108, -8), (-100, -20)])
+def test_f16w3_small_results(ta, ex, ea, eb):
+    """Whole pieces whose products are near f32's smallest normal: f32 sums
+    of K products in any order, and the rounding of denormals."""
+    rng = np.random.default_rng(10)
+    m, n, k = 40, 72, 200
+    a = np.ldexp(rng.uniform(1, 2, (m, k)), ea).astype(np.float32)
+    b = np.ldexp(rng.uniform(1, 2, (k, n)), eb).astype(np.float16).astype(np.float32)
+    c = ex.tensor([m, n])
+    ex.run_ops([ta.MatmulOp(ex.tensor_from(a), ex.tensor_from(b, f16=True), c)])
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    # five piece products of each pair round to multiples of 2^-149
+    assert np.all(np.abs(ex.download(c) - exact) <= k * (2.0 ** -24 * exact + 5 * 2.0 ** -150))
+
+
 @pytest.mark.parametrize("bt,m,n,k", [(1, 33, 65, 1000), (1, 63, 136, 161), (1, 9, 8, 4096), (3, 8, 130, 513), (2, 40, 72, 2800)])
 @pytest.mark.parametrize("special", ["a", "b"])
 def test_f16w3_whole_f32_tiles(ta, ex, oracle, bt, m, n, k, special):
