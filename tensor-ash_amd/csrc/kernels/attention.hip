@@ -42,10 +42,11 @@ template <int DH> constexpr int flash_qblocks() { return ta_flash_qblocks(DH); }
 constexpr float kNegMax = -3.402823466e38f;
 constexpr float kMasked = -__builtin_inff();
 constexpr float kMinScale = 1.17549435e-38f; // 2^-126
-// f16-cache kernels: a row's reference point (m_run) lies kProbBits below a
-// maximum of its scores, so that its probabilities, at most 2^(kProbBits +
-// kSlack), use the range of their f16 pieces.
-constexpr float kProbBits = 11.0f, kSlack = 4.0f;
+// f16-cache kernels: a row's probabilities stay below 2^kSlack and are scaled
+// by kProbScale, so that they use the range of their f16 pieces.  (A
+// reference point 11 below the maximum would scale them too, but rounds the
+// exponents of the largest ones to 2^-21: 2.2e-7 off instead of 1.9e-7.)
+constexpr float kSlack = 4.0f, kProbScale = 2048.0f;
 // What the first piece of an f32 operand leaves over is scaled by kLowScale
 // before it becomes f16, and its products are summed apart.
 constexpr float kLowScale = 2048.0f;
@@ -417,16 +418,18 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 //  * q: as it is when f16; f32 rows are scaled by a power of two (largest
 //    value into [2^14, 2^15)) and split into three pieces: exactly down to
 //    2^-26 of the row's largest value, to 2^-50 of it below that;
-//  * probabilities: two pieces, within 2^-24 of every value down to 2^-23 of
+//  * probabilities: two pieces, within 2^-23 of every value down to 2^-23 of
 //    the row's largest, and to 2^-47 of that below; the row sum takes the f32
 //    values.
 // The pieces after the first are scaled by kLowScale and summed apart: in one
 // sum they end at f16's smallest step, 2^-36 of a row's largest probability
 // and 2^-40 of its largest q, and results that come from keys of 2^-26 alone
-// were 8e-4 off (now 6e-7).  It costs 16 FMAs a tile and 32 columns: 76.6 ->
-// 80.5 us at the first size below, 31.8 -> 35.8 for 16 heads of dh 64.
-// Measured against f64 (normal inputs): 1.7e-7 .. 3.5e-7, as the f32 MFMA
-// kernel had.  An infinite operand would meet zero pieces (inf * 0); rows
+// were 8e-4 off (now 6e-7).  It costs 5 to 8%, by keeping their sums apart to
+// the end at dh 64 (16 FMAs a tile and 32 columns instead: 37.0 us for 33.7,
+// 2048 tokens, 16 / 4 heads, in one sum 32.0); at dh 128 there are no
+// registers for that.
+// Measured against f64 (normal inputs): 1.2e-7 .. 2.1e-7 (in one sum 1.5e-7 ..
+// 2.7e-7).  An infinite operand would meet zero pieces (inf * 0); rows
 // that come out non-finite are computed again by flash_rows_whole.
 //
 // Layout.  K and V tiles stay in LDS as they lie in the caches ([d][key],
@@ -444,8 +447,8 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 // wave; ta_flash16_rows).  Tiles of 128 rows x 64 keys were slower (102
 // against 94 us): fewer, longer workgroups leave CUs idle at the end.
 //
-// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 80.5
-// us here (427 TFLOP/s), kv16 434 -> 112 us; 512 tokens, 4 KV heads, dh 64,
+// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 82 us
+// here (420 TFLOP/s), kv16 434 -> 114 us; 512 tokens, 4 KV heads, dh 64,
 // f16: 28 -> 10.9 us.  MFMAs are busy 30% (kv16 38%) and CUs 75%; a wave's
 // scores, softmax and PV product follow each other and overlap only with its
 // SIMD's other wave.
@@ -568,10 +571,16 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
       for (int s = 0; s < KS; ++s)
         asm volatile("" : "+v"(qf[q][s]));
 
-    f32x16 o[DB];
+    // The smaller pieces' sums: kept apart to the end, or added tile by tile
+    // where that many registers would cost a workgroup.
+    constexpr bool APART = DH == 64;
+    f32x16 o[DB], o_low[APART ? DB : 1];
 #pragma unroll
-    for (int b = 0; b < DB; ++b)
+    for (int b = 0; b < DB; ++b) {
       o[b] = f32x16{};
+      if constexpr (APART)
+        o_low[b] = f32x16{};
+    }
     float m_run = kNegMax, l_run = 0.0f;
 
     const _Float16 *kt = static_cast<const _Float16 *>(p.kt) + (uint64_t)kv_head * DH * p.t_max;
@@ -736,16 +745,19 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
       // by 2^kSlack (probabilities stay below 2^kSlack): with 32 rows in a
       // wave some row finds a new maximum in nearly every tile, and scaling
       // the output for it was a third of the softmax's instructions.
-      if (__any(tmax > m_run + (kProbBits + kSlack))) {
-        const float m_new = fmaxf(m_run, tmax - kProbBits);
+      if (__any(tmax > m_run + kSlack)) {
+        const float m_new = fmaxf(m_run, tmax);
         const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
         l_run *= corr;
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
-          for (int e = 0; e < 16; ++e)
+          for (int e = 0; e < 16; ++e) {
             o[b][e] *= corr;
+            if constexpr (APART)
+              o_low[b][e] *= corr;
+          }
       }
       float psum = 0.0f;
 #pragma unroll
@@ -754,7 +766,7 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
         for (int e = 0; e < 16; ++e) {
           const float pv = __builtin_amdgcn_exp2f(fmaf(s[kb][e], scale2, -m_run));
           psum += pv;
-          s[kb][e] = pv;
+          s[kb][e] = pv * kProbScale;
         }
       l_run += psum;
 
@@ -779,6 +791,8 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
 #pragma unroll
       for (int b = 0; b < DB; ++b) {
         f32x16 low = f32x16{};
+        if constexpr (APART)
+          low = o_low[b];
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -788,13 +802,24 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
             o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi[kb][u], o[b], 0, 0, 0);
             low = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo[kb][u], low, 0, 0, 0);
           }
+        if constexpr (APART) {
+          o_low[b] = low;
+        } else {
 #pragma unroll
-        for (int e = 0; e < 16; ++e)
-          o[b][e] = fmaf(low[e], 1.0f / kLowScale, o[b][e]);
+          for (int e = 0; e < 16; ++e)
+            o[b][e] = fmaf(low[e], 1.0f / kLowScale, o[b][e]);
+        }
       }
       if (t + 1 < n_tiles)
         commit(t + 1);
     }
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        o[b][e] = (APART ? fmaf(o_low[APART ? b : 0][e], 1.0f / kLowScale, o[b][e]) : o[b][e]) *
+                  (1.0f / kProbScale);
+
     float m = m_run, l = l_run, a0 = 1.0f;
     float mp[KP], a[KP];
     float *mb = reinterpret_cast<float *>(smem) + qb * ((KP - 1) * REGS * 64);
