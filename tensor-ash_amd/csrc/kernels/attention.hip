@@ -424,10 +424,11 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 // The pieces after the first are scaled by kLowScale and summed apart: in one
 // sum they end at f16's smallest step, 2^-36 of a row's largest probability
 // and 2^-40 of its largest q, and results that come from keys of 2^-26 alone
-// were 8e-4 off (now 6e-7).  It costs 5 to 8%, by keeping their sums apart to
-// the end at dh 64 (16 FMAs a tile and 32 columns instead: 37.0 us for 33.7,
-// 2048 tokens, 16 / 4 heads, in one sum 32.0); at dh 128 there are no
-// registers for that.
+// were 8e-4 off (now 6e-7).  At dh 64 their sums stay apart to the end (2048
+// tokens, 16 / 4 heads: 32.9 us, in one sum 32.3); at dh 128 there are no
+// registers for that, and 64 FMAs a tile add them (82 us, in one sum 77, at
+// the size below; two columns' blocks at a time, or the smaller products
+// first, were no faster).
 // Measured against f64 (normal inputs): 1.2e-7 .. 2.1e-7 (in one sum 1.5e-7 ..
 // 2.7e-7).  An infinite operand would meet zero pieces (inf * 0); rows
 // that come out non-finite are computed again by flash_rows_whole.
@@ -788,23 +789,33 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
             lo[kb][u][e] = (_Float16)fmaf((float)a[0], -kLowScale, x * kLowScale);
             lo[kb][u][e + 1] = (_Float16)fmaf((float)a[1], -kLowScale, y * kLowScale);
           }
-#pragma unroll
-      for (int b = 0; b < DB; ++b) {
-        f32x16 low = f32x16{};
-        if constexpr (APART)
-          low = o_low[b];
+      auto v_at = [&](int b, int kb, int u) __attribute__((always_inline)) {
+        const uint32_t at = st + v_off[b] + (kb * 32 + u * 16) * (DH * 2);
+        return tr(at, at + 8 * (DH * 2));
+      };
+      if constexpr (APART) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const uint32_t at = st + v_off[b] + (kb * 32 + u * 16) * (DH * 2);
-            const f16x8 a = tr(at, at + 8 * (DH * 2));
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi[kb][u], o[b], 0, 0, 0);
-            low = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo[kb][u], low, 0, 0, 0);
-          }
-        if constexpr (APART) {
-          o_low[b] = low;
-        } else {
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int b = 0; b < DB; ++b) {
+              const f16x8 a = v_at(b, kb, u);
+              o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi[kb][u], o[b], 0, 0, 0);
+              o_low[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo[kb][u], o_low[b], 0, 0, 0);
+            }
+      } else {
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+          f32x16 low = f32x16{};
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const f16x8 a = v_at(b, kb, u);
+              o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi[kb][u], o[b], 0, 0, 0);
+              low = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo[kb][u], low, 0, 0, 0);
+            }
 #pragma unroll
           for (int e = 0; e < 16; ++e)
             o[b][e] = fmaf(low[e], 1.0f / kLowScale, o[b][e]);
