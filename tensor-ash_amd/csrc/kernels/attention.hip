@@ -541,9 +541,10 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
               qmax = fmaxf(qmax, fabsf(raw[s][i][c]));
           }
         qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
-        // largest |q| of the row into [2^14, 2^15)
+        // largest |q| of the row into [2^14, 2^15); the factor ends at 2^127,
+        // which leaves rows below 2^-112 as exact (f32's denormals end there)
         int e = 15 - __builtin_amdgcn_frexp_expf(qmax);
-        e = qmax > 0.0f ? min(max(e, -100), 100) : 0;
+        e = qmax > 0.0f ? min(e, 127) : 0;
         const float up = ldexpf(sign, e);
         scale2 = scale2 * ldexpf(1.0f, -e);
 #pragma unroll

@@ -357,6 +357,25 @@ def test_flash_f16_cache_light_keys(ta, ex, dh, io16):
 
 
 @pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("ea", [-125, -114, -60, 60, 120])
+def test_flash_f16_cache_q_of_any_size(ta, ex, oracle, dh, ea):
+    """f32 q of any magnitude, with a scale that brings the scores back: the
+    result of the same q at 1."""
+    heads, t = 2, 70
+    q = oracle.fill_det(heads * t * dh, 5830).reshape(heads, t, dh)
+    kt, v = fill_kv(oracle, heads, dh, t, t)
+    kt, v = oracle.round_via_f16(kt).reshape(kt.shape), oracle.round_via_f16(v).reshape(v.shape)
+    q = np.ldexp(np.ldexp(q, ea), -ea)  # as f32's denormals round it
+    out = ex.tensor([heads, t, dh])
+    ex.flash_attention(ex.tensor_from(np.ldexp(q, ea)), ex.tensor_from(kt, f16=True), ex.tensor_from(v, f16=True), out,
+                       ta.FlashAttentionDesc(t, 0, float(np.ldexp(0.5, -ea))))
+    ref = oracle.flash_attention(q, kt, v, heads, heads, t, t, dh, t, 0, 0.5)
+    err, idx = oracle.max_abs_err(ex.download(out).reshape(-1), ref)
+    print(f"error {err:.2e}", flush=True)
+    assert err <= 2e-5, f"err {err} at {idx}"
+
+
+@pytest.mark.parametrize("dh", [64, 128])
 def test_flash_f16_cache_q_over_a_wide_range(ta, ex, oracle, dh):
     """f32 q whose largest value meets zeros of K: scores come from values
     2^-27 of it, and stay exact products (2^-40 of the largest alone would
