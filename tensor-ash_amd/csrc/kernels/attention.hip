@@ -424,11 +424,11 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 // The pieces after the first are scaled by kLowScale and summed apart: in one
 // sum they end at f16's smallest step, 2^-36 of a row's largest probability
 // and 2^-40 of its largest q, and results that come from keys of 2^-26 alone
-// were 8e-4 off (now 6e-7).  At dh 64 their sums stay apart to the end (2048
-// tokens, 16 / 4 heads: 32.9 us, in one sum 32.3); at dh 128 there are no
-// registers for that, and 64 FMAs a tile add them (82 us, in one sum 77, at
-// the size below; two columns' blocks at a time, or the smaller products
-// first, were no faster).
+// were 8e-4 off (now 6e-7).  Where the registers are there (dh 64; dh 128 with
+// f16 q and 64 rows) their sums stay apart to the end: 2048 tokens, 16 / 4
+// heads of dh 64 32.9 us (in one sum 32.3), the size below 78 (76).  Else they
+// are added tile by tile, 64 FMAs at dh 128 (f32 q 113 us for 106; kept apart
+// it spills, 170).
 // Measured against f64 (normal inputs): 1.2e-7 .. 2.1e-7 (in one sum 1.5e-7 ..
 // 2.7e-7).  An infinite operand would meet zero pieces (inf * 0); rows
 // that come out non-finite are computed again by flash_rows_whole.
@@ -448,9 +448,9 @@ template <int DH> TA_DEVICE void flash_body(const FlashArgs &p) {
 // wave; ta_flash16_rows).  Tiles of 128 rows x 64 keys were slower (102
 // against 94 us): fewer, longer workgroups leave CUs idle at the end.
 //
-// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 82 us
-// here (420 TFLOP/s), kv16 434 -> 114 us; 512 tokens, 4 KV heads, dh 64,
-// f16: 28 -> 10.9 us.  MFMAs are busy 30% (kv16 38%) and CUs 75%; a wave's
+// 2048 tokens, 32 heads / 8 KV, dh 128, f16: 437 us on the f32 MFMAs, 78 us
+// here (440 TFLOP/s), kv16 434 -> 113 us; 512 tokens, 4 KV heads, dh 64,
+// f16: 28 -> 10.9 us.  MFMAs are busy 32% (kv16 37%) and CUs 75%; a wave's
 // scores, softmax and PV product follow each other and overlap only with its
 // SIMD's other wave.
 template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH16 {
@@ -574,8 +574,9 @@ template <int DH, bool IO16, bool DIRECT, int QB, int KP, int BKW> struct FlashH
         asm volatile("" : "+v"(qf[q][s]));
 
     // The smaller pieces' sums: kept apart to the end, or added tile by tile
-    // where that many registers would cost a workgroup.
-    constexpr bool APART = DH == 64;
+    // where there are no registers for that (the two round alike, not the
+    // same: f16 q and the same q in f32 may differ in an f16 result's last bit).
+    constexpr bool APART = DH == 64 || (QB == 2 && IO16);
     f32x16 o[DB], o_low[APART ? DB : 1];
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
